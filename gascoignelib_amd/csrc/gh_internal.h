@@ -15,19 +15,32 @@
 
 #include "gascoigne_hip.h"
 
-// Vanka patch smoother: patch LU factors and the node -> patch lists
+// Vanka patch smoother: patch LU factors and the node -> patch lists.  Patches
+// with the same matrix, bit for bit, share one set of factors (a class): on a
+// uniformly refined mesh with constant coefficients a few dozen classes serve
+// all patches.
 struct gh_vanka {
   gh_ctx* ctx = nullptr;
   int B = 1, psize = 0, m = 0;
   int prec = GH_F64;          // storage of the factors and of the local solves
   int64_t n = 0, npatches = 0;
+  int64_t nclasses = 0;       // distinct patch matrices
+  int ld = 0;                 // entries of a factor column: m rounded up to 16, zeros below row m
+  int64_t lstride = 0;        // entries of one class's factors: ld * m
   int32_t* nodes = nullptr;   // npatches * psize
-  void* lu = nullptr;         // npatches * m * m, column-major, L unit lower
-  int32_t* piv = nullptr;     // npatches * m: row exchanges, then (after set-up) the
-                              // global entry gathered into each factor row
+  int32_t* cls = nullptr;     // class of each patch
+  void* lu = nullptr;         // nclasses * lstride, column-major, L unit lower
+  double* rdiag = nullptr;    // nclasses * m: 1 / u_kk, 0 where it is not used
+  int32_t* piv = nullptr;     // npatches * m: the global entry gathered into each factor row
   int32_t* nptr = nullptr;    // n + 1
   int32_t* nent = nullptr;    // patch * psize + local node, ascending patch per node
   void* xp = nullptr;         // npatches * m local solutions
+  // grouped solve: workgroup g takes the patches plist[first .. first + count)
+  // of one class; (class, first, count) per group.  ngroups = 0: one wavefront
+  // per patch instead
+  int64_t ngroups = 0;
+  int32_t* groups = nullptr;
+  int32_t* plist = nullptr;
 };
 
 // Q1 box cells for coefficient gradients
@@ -320,7 +333,10 @@ int csr_residual(gh_ctx* ctx, const gh_csr* A, int prec, void* r, const void* x,
 int csr_spmv_x32(gh_ctx* ctx, const gh_csr* A, double* y, const float* x);
 int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, const int32_t* nodes,
                  int prec, gh_vanka** out);
-int vanka_solve(gh_ctx* ctx, const gh_vanka* V, int prec, void* x);
+// VankaSmoother::solve of `in`: mode 0 out = h, 1 out += omega h, 2 out = omega h
+// (`in` and `out` may alias in mode 0)
+int vanka_apply(gh_ctx* ctx, const gh_vanka* V, int prec, const void* in, void* out, int mode,
+                double omega);
 // the inverse of an FP64 matrix (scalar or node blocks) as a dense row-major
 // m x m array on the device (m = n * ncomp), factorised on the device
 int dense_inverse_device(gh_ctx* ctx, const gh_csr* A, double* inv);

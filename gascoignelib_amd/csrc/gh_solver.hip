@@ -283,23 +283,14 @@ int sweep(gh_mg* mg, MgLevel& L, int niter, bool& u_zero, void* keep_u) {
     if (niter > 0 && vanka && !L.vanka) return fail(GH_EINVAL, "vanka smoother: level without patches");
     if (niter > 0 && !vanka && !L.ilu) return fail(GH_EINVAL, "ilu smoother: level without factors");
     for (int it = 0; it < niter; ++it) {
-      if (!vanka) {
-        // the ILU solve reads h through its order and adds omega h to x itself
-        if (!u_zero) GH_TRY(csr_residual(mg->ctx, L.A, mg->wprec, L.v, L.u, L.b));
-        GH_TRY(ilu_apply(mg->ctx, L.ilu, mg->wprec, u_zero ? L.b : L.v, L.u, u_zero ? 2 : 1,
-                         mg->P.omega));
-        u_zero = false;
-        continue;
-      }
-      if (u_zero)
-        GH_TRY(vec_convert(mg->ctx, L.size, mg->wprec, L.v, mg->wprec, L.b));
+      // the solves read h through their gather and add omega h to x themselves
+      if (!u_zero) GH_TRY(csr_residual(mg->ctx, L.A, mg->wprec, L.v, L.u, L.b));
+      const void* h = u_zero ? L.b : L.v;
+      const int mode = u_zero ? 2 : 1;
+      if (vanka)
+        GH_TRY(vanka_apply(mg->ctx, L.vanka, mg->wprec, h, L.u, mode, mg->P.omega));
       else
-        GH_TRY(csr_residual(mg->ctx, L.A, mg->wprec, L.v, L.u, L.b));
-      GH_TRY(vanka_solve(mg->ctx, L.vanka, mg->wprec, L.v));
-      if (u_zero)
-        GH_TRY(vec_scale_to(mg->ctx, mg->wprec, L.size, L.u, mg->P.omega, L.v));
-      else
-        GH_TRY(vec_axpby(mg->ctx, mg->wprec, L.size, L.u, 1.0, mg->P.omega, L.v));
+        GH_TRY(ilu_apply(mg->ctx, L.ilu, mg->wprec, h, L.u, mode, mg->P.omega));
       u_zero = false;
     }
     (void)keep_u;

@@ -4,12 +4,13 @@
 // Factoring: one workgroup of 1024 threads per patch, the m x m patch matrix
 // (m <= 128) in the threads' registers, the LU's operations uncontracted so
 // that the factors equal the oracle's; the recorded row exchanges are composed on the host into
-// one gather per factor row.  Solving: one wavefront per patch, the local vector
-// gathered in pivoted order into the lanes' registers (rows lane and
-// lane + 64), column-oriented triangular solves (each pass reads only its
-// triangle) with the solved values broadcast by readlane.  Averaging: one
-// thread per unknown, the patches containing its node added in ascending order
-// (the reference adds with OpenMP atomics, in no fixed order).
+// one gather per factor row.  Patches with equal matrices are found first and
+// factored once.  Solving: column-oriented triangular solves of the local
+// vector, gathered in pivoted order, by one of two kernels: grouped (the
+// factors of one class in LDS, 16 lanes per patch, k_vanka_group) or streamed
+// (one wavefront per patch reading its own factors, k_vanka_solve).  Averaging:
+// one thread per unknown, the patches containing its node added in ascending
+// order (the reference adds with OpenMP atomics, in no fixed order).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -175,41 +176,113 @@ __device__ __forceinline__ void factor_columns(int m, int tr, int tc,
   }
 }
 
-// LU with partial pivoting of every patch matrix, the oracle's operations in
+// copy_entries_sparseblockmatrix: tab[r * psize + u] = CSR position of the block
+// (patch node r, patch node u), -1 where the matrix has none.  All NT threads of
+// the workgroup; NT / psize of them walk each row's entries.  Ends in a barrier.
+template <int NT>
+__device__ __forceinline__ void patch_positions(int psize, const int32_t* __restrict__ nodes,
+                                                const int32_t* __restrict__ rowptr,
+                                                const int32_t* __restrict__ col, int32_t* tab,
+                                                int32_t* pn) {
+  const int t = threadIdx.x;
+  for (int e = t; e < psize * psize; e += NT) tab[e] = -1;
+  for (int r = t; r < psize; r += NT) pn[r] = nodes[r];
+  __syncthreads();
+  const int per = NT / psize;
+  const int r = t / per, u0 = t - r * per;
+  if (r < psize) {
+    const int32_t row = pn[r];
+    for (int32_t q = rowptr[row] + u0; q < rowptr[row + 1]; q += per) {
+      const int32_t c0 = col[q];
+      for (int u = 0; u < psize; ++u)
+        if (pn[u] == c0) tab[r * psize + u] = q;
+    }
+  }
+  __syncthreads();
+}
+
+// the 64-bit finaliser of SplitMix64
+__device__ __forceinline__ uint64_t mix64(uint64_t z) {
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+
+constexpr int kHashThreads = 256;
+
+// Two 64-bit sums over the patch matrix's entries, each entry's bits mixed with
+// its place: equal matrices have equal sums, and the patches with equal sums are
+// compared entry by entry afterwards (k_vanka_same).
+__global__ __launch_bounds__(kHashThreads) void k_vanka_hash(
+    int psize, int B, const int32_t* __restrict__ nodes, const int32_t* __restrict__ rowptr,
+    const int32_t* __restrict__ col, const double* __restrict__ val, uint64_t* __restrict__ out) {
+  extern __shared__ int32_t tab[];
+  __shared__ int32_t pn[kVankaMaxNodes];
+  __shared__ uint64_t part[2][kHashThreads / 64];
+  const int64_t p = blockIdx.x;
+  const int BB = B * B, t = threadIdx.x;
+  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, pn);
+  uint64_t h0 = 0, h1 = 0;
+  for (int e = t; e < psize * psize * BB; e += kHashThreads) {
+    const int32_t q = tab[e / BB];
+    const double x = q >= 0 ? val[(int64_t)q * BB + e % BB] : 0.0;
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    h0 += mix64(b + (uint64_t)(e + 1) * 0x9E3779B97F4A7C15ull);
+    h1 += mix64((b ^ 0xD1B54A32D192ED03ull) + (uint64_t)(e + 1) * 0xABC98388FB8FAC03ull);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    h0 += (uint64_t)__shfl_down((unsigned long long)h0, off, 64);
+    h1 += (uint64_t)__shfl_down((unsigned long long)h1, off, 64);
+  }
+  if ((t & 63) == 0) {
+    part[0][t >> 6] = h0;
+    part[1][t >> 6] = h1;
+  }
+  __syncthreads();
+  if (t < 2) {
+    uint64_t s = 0;
+    for (int w = 0; w < kHashThreads / 64; ++w) s += part[t][w];
+    out[2 * p + t] = s;
+  }
+}
+
+// flag[p] = 1 where patch p's matrix differs from patch rep[p]'s in any bit
+__global__ __launch_bounds__(kHashThreads) void k_vanka_same(
+    int psize, int B, const int32_t* __restrict__ nodes, const int32_t* __restrict__ rowptr,
+    const int32_t* __restrict__ col, const double* __restrict__ val,
+    const int32_t* __restrict__ rep, int32_t* __restrict__ flag) {
+  extern __shared__ int32_t tab[];  // 2 * psize * psize
+  __shared__ int32_t pn[kVankaMaxNodes];
+  const int64_t p = blockIdx.x, r = rep[p];
+  if (r == p) return;  // the whole workgroup
+  const int BB = B * B, PP = psize * psize;
+  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, pn);
+  patch_positions<kHashThreads>(psize, nodes + r * psize, rowptr, col, tab + PP, pn);
+  for (int e = threadIdx.x; e < PP * BB; e += kHashThreads) {
+    const int32_t q = tab[e / BB], s = tab[PP + e / BB];
+    const double x = q >= 0 ? val[(int64_t)q * BB + e % BB] : 0.0;
+    const double y = s >= 0 ? val[(int64_t)s * BB + e % BB] : 0.0;
+    if (__builtin_bit_cast(uint64_t, x) != __builtin_bit_cast(uint64_t, y)) flag[p] = 1;
+  }
+}
+
+// LU with partial pivoting of every class's patch matrix, the oracle's operations in
 // the oracle's order per entry: pivot = the first row (in the exchanged order)
 // of largest |a_ik|, i >= k; no elimination when the pivot is 0;
 // l_i = a_ik / d and a_ij -= l_i a_kj, product and difference rounded
 // separately.  (8 waves per SIMD: two patches per CU, at most 64 VGPRs.)
 __global__ __launch_bounds__(kFactorThreads, 8) void k_vanka_factor(
-    int64_t npatches, int psize, int B, const int32_t* __restrict__ nodes,
+    int psize, int B, const int32_t* __restrict__ reps, const int32_t* __restrict__ nodes,
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-    const double* __restrict__ val, double* __restrict__ lu64, float* __restrict__ lu32,
-    int32_t* __restrict__ piv) {
+    const double* __restrict__ val, int ld, double* __restrict__ lu64,
+    float* __restrict__ lu32, int32_t* __restrict__ piv) {
   extern __shared__ int32_t tab[];  // psize * psize CSR positions of the node blocks, -1: none
   __shared__ int32_t pn[kVankaMaxNodes];
   __shared__ FactorShared S;
-  constexpr int NT = kFactorThreads;
   const int64_t p = blockIdx.x;
   const int m = psize * B;
   const int t = threadIdx.x, tr = t % kFactorLanes, tc = t / kFactorLanes;
-  for (int e = t; e < psize * psize; e += NT) tab[e] = -1;
-  for (int r = t; r < psize; r += NT) pn[r] = nodes[p * psize + r];
-  __syncthreads();
-  // copy_entries_sparseblockmatrix: the entries whose column is a patch node.
-  // NT / psize threads (at least 8) walk each row's entries.
-  {
-    const int per = NT / psize;
-    const int r = t / per, u0 = t - r * per;
-    if (r < psize) {
-      const int32_t row = pn[r];
-      for (int32_t q = rowptr[row] + u0; q < rowptr[row + 1]; q += per) {
-        const int32_t c0 = col[q];
-        for (int u = 0; u < psize; ++u)
-          if (pn[u] == c0) tab[r * psize + u] = q;
-      }
-    }
-  }
-  __syncthreads();
+  patch_positions<kFactorThreads>(psize, nodes + (int64_t)reps[p] * psize, rowptr, col, tab, pn);
   double a[kRowsPer][kColsPer];
   int pos[kRowsPer];  // position of row tr + 64 i in the exchanged order; -1: no row
 #pragma unroll
@@ -238,7 +311,7 @@ __global__ __launch_bounds__(kFactorThreads, 8) void k_vanka_factor(
   factor_columns<7>(m, tr, tc, a, pos, S, pv);
   // column-major factors (coalesced column reads in the solve), rows in the
   // exchanged order
-  const int64_t base = p * (int64_t)m * m;
+  const int64_t base = p * (int64_t)ld * m;
 #pragma unroll
   for (int i = 0; i < kRowsPer; ++i) {
     if (pos[i] < 0) continue;
@@ -246,7 +319,7 @@ __global__ __launch_bounds__(kFactorThreads, 8) void k_vanka_factor(
     for (int j = 0; j < kColsPer; ++j) {
       const int c = tc + kFactorWaves * j;
       if (c >= m) continue;
-      const int64_t e = base + (int64_t)c * m + pos[i];
+      const int64_t e = base + (int64_t)c * ld + pos[i];
       if (lu64) lu64[e] = a[i][j];
       else lu32[e] = (float)a[i][j];
     }
@@ -268,6 +341,7 @@ __device__ __forceinline__ T bcast(T v, int lane) {
 // one wavefront per patch; rows lane (slot 0) and lane + 64 (slot 1)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int psize, int B,
+                                                        const int32_t* __restrict__ cls, int ld,
                                                         const T* __restrict__ lu,
                                                         const int32_t* __restrict__ gidx,
                                                         const T* __restrict__ h,
@@ -276,7 +350,7 @@ __global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int ps
   const int64_t p = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (p >= npatches) return;  // the whole wavefront
   const int m = psize * B;
-  const T* L = lu + p * (int64_t)m * m;
+  const T* L = lu + (int64_t)cls[p] * ld * m;
   // H = P H: gidx holds, per row of the factors, the global entry that the
   // recorded row exchanges bring there
   const int32_t* gi = gidx + p * m;
@@ -298,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int ps
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int k = min(k0 + u, m - 1);
-      const T* Lk = L + (int64_t)k * m;
+      const T* Lk = L + (int64_t)k * ld;
       a0[u] = (in0 && lane > k) ? Lk[lane] : (T)0;
       a1[u] = (in1 && lane + 64 > k) ? Lk[lane + 64] : (T)0;
     }
@@ -318,7 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int ps
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int kk = max(k0 - u, 0);
-      const T* Uk = L + (int64_t)kk * m;
+      const T* Uk = L + (int64_t)kk * ld;
       a0[u] = lane < kk ? Uk[lane] : (T)0;
       a1[u] = lane + 64 < kk ? Uk[lane + 64] : (T)0;
       dg[u] = Uk[kk];
@@ -342,13 +416,285 @@ __global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int ps
   if (lane + 64 < m) out[lane + 64] = v1;
 }
 
-// x(i, c) = (sum over the patches of node i, ascending) * (1 / count_i)
+// ------------------------------------------------------------ grouped solve
+// reciprocals of the diagonal of U for the grouped solve's divisions; 0 where
+// a plain division is needed (zero or extreme diagonals)
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_vanka_rdiag(int64_t nclasses, int m, int ld,
+                                                        const T* __restrict__ lu,
+                                                        double* __restrict__ rdiag) {
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (t >= nclasses * m) return;
+  const int64_t c = t / m;
+  const int k = (int)(t - c * m);
+  const double d = (double)lu[(c * m + k) * ld + k];
+  const double a = fabs(d);
+  rdiag[t] = (a >= 0x1p-400 && a <= 0x1p400) ? 1.0 / d : 0.0;
+}
+
+// x / d rounded to nearest, r = 1 / d rounded to nearest.  FP64: two residual
+// corrections of x r (P. Markstein, IBM J. Res. Dev. 34 (1990): with r correctly
+// rounded and q within an ulp of x / d, fma(x - q d, r, q) is x / d correctly
+// rounded), 5 dependent operations; up to the sign of a zero the quotients are
+// the division's, so the solves keep the oracle's values.  FP32: the product
+// with the FP64 reciprocal.
+__device__ __forceinline__ double divide_by(double x, double d, double r) {
+  const double q0 = x * r;
+  const double q1 = __builtin_fma(__builtin_fma(-q0, d, x), r, q0);
+  return __builtin_fma(__builtin_fma(-q1, d, x), r, q1);
+}
+__device__ __forceinline__ float divide_by(float x, double, double r) {
+  return (float)((double)x * r);
+}
+// whether the quotient q of divide_by, by a diagonal within 2^-400 .. 2^400,
+// was free of overflow and underflow on the way (then x was within 2^+-700)
+__device__ __forceinline__ bool in_range(double q) {
+  const double a = fabs(q);
+  return (a >= 0x1p-300 && a <= 0x1p300) || a == 0.0;
+}
+__device__ __forceinline__ bool in_range(float q) { return fabsf(q) <= 3.0e38f; }
+
+// lane N of each 16-lane row, to the whole row
+template <int N>
+__device__ __forceinline__ float row_bcast(float x) {
+  const int b = __builtin_bit_cast(int, x);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x150 + N, 0xf, 0xf, false));
+}
+template <int N>
+__device__ __forceinline__ double row_bcast(double x) {
+  const int64_t b = __builtin_bit_cast(int64_t, x);
+  const int l = (int)(b & 0xFFFFFFFF), h = (int)(b >> 32);
+  const int lo = __builtin_amdgcn_update_dpp(l, l, 0x150 + N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(h, h, 0x150 + N, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((int64_t)hi << 32) | (uint32_t)lo);
+}
+
+// The passes go in sets of kSet columns: the next set's factors are read from
+// LDS before this set's steps, and no read or address moves further (the
+// compiler would otherwise hoist all of them and spill).  v[j] is the lane's
+// row 16 j + r, r = lane % 16.
+template <typename T> constexpr int kSet = sizeof(T) == 8 ? 2 : 4;
+__device__ __forceinline__ void reads_stay(int& r) {
+  asm volatile("" : "+v"(r)::"memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// columns S kSet .. S kSet + kSet - 1, rows from the diagonal's 16 down
+template <int MB, int S, typename T>
+__device__ __forceinline__ void load_lower(const T* __restrict__ L, int r, T (&c)[kSet<T>][MB]) {
+#pragma unroll
+  for (int s = 0; s < kSet<T>; ++s) {
+    const int k = S * kSet<T> + s;
+#pragma unroll
+    for (int j = k / 16; j < MB; ++j) c[s][j] = L[r + k * 16 * MB + 16 * j];
+  }
+}
+// forward step (unit lower triangle): column k updates the rows below k
+template <int MB, int K, typename T>
+__device__ __forceinline__ void step_lower(const T (&c)[MB], int r, T (&v)[MB]) {
+  constexpr int KB = K / 16, N = K % 16;
+  const T y = row_bcast<N>(v[KB]);
+  if constexpr (N < 15) {
+    const T u = add_rn(v[KB], -mul_rn(c[KB], y));
+    v[KB] = r > N ? u : v[KB];
+  }
+#pragma unroll
+  for (int j = KB + 1; j < MB; ++j) v[j] = add_rn(v[j], -mul_rn(c[j], y));
+}
+template <int MB, int S, typename T>
+__device__ __forceinline__ void group_forward(const T* __restrict__ L, int r, T (&v)[MB],
+                                              const T (&c)[kSet<T>][MB]) {
+  constexpr int Q = kSet<T>, K = S * Q;
+  T next[Q][MB];
+  if constexpr (K + Q < 16 * MB) load_lower<MB, S + 1>(L, r, next);
+  reads_stay(r);
+  step_lower<MB, K>(c[0], r, v);
+  step_lower<MB, K + 1>(c[1], r, v);
+  if constexpr (Q == 4) {
+    step_lower<MB, K + 2>(c[2], r, v);
+    step_lower<MB, K + 3>(c[3], r, v);
+  }
+  if constexpr (K + Q < 16 * MB) group_forward<MB, S + 1>(L, r, v, next);
+}
+
+template <typename T, int MB>
+struct UpperSet {
+  T c[kSet<T>][MB];
+  double d[kSet<T>], rk[kSet<T>];  // u_kk and its reciprocal
+};
+// columns S kSet .. S kSet + kSet - 1, rows up to the diagonal's 16
+template <int MB, int S, typename T>
+__device__ __forceinline__ void load_upper(const T* __restrict__ L, int r,
+                                           const double* __restrict__ rd, UpperSet<T, MB>& u) {
+#pragma unroll
+  for (int s = 0; s < kSet<T>; ++s) {
+    const int k = S * kSet<T> + s;
+#pragma unroll
+    for (int j = 0; j <= k / 16; ++j) u.c[s][j] = L[r + k * 16 * MB + 16 * j];
+    u.d[s] = rd[2 * k];
+    u.rk[s] = rd[2 * k + 1];
+  }
+}
+// backward step: y_k = v_k / u_kk, then column k updates the rows above k.
+// Rows and columns past the matrix are zeros in LDS (u_kk = 1) and stay zero.
+template <int MB, int K, typename T>
+__device__ __forceinline__ void step_upper(const T (&c)[MB], double d, double rk, int r,
+                                           T (&v)[MB]) {
+  constexpr int KB = K / 16, N = K % 16;
+  const T q = divide_by(v[KB], d, rk);
+  const T y = row_bcast<N>(q);
+  const T u = add_rn(v[KB], -mul_rn(c[KB], y));
+  v[KB] = r < N ? u : (r == N ? q : v[KB]);
+#pragma unroll
+  for (int j = 0; j < KB; ++j) v[j] = add_rn(v[j], -mul_rn(c[j], y));
+}
+template <int MB, int S, typename T>
+__device__ __forceinline__ void group_backward(const T* __restrict__ L,
+                                               const double* __restrict__ rd, int r,
+                                               T (&v)[MB], const UpperSet<T, MB>& u) {
+  constexpr int Q = kSet<T>, K = S * Q;
+  UpperSet<T, MB> next;
+  if constexpr (S > 0) load_upper<MB, S - 1>(L, r, rd, next);
+  reads_stay(r);
+  if constexpr (Q == 4) {
+    step_upper<MB, K + 3>(u.c[3], u.d[3], u.rk[3], r, v);
+    step_upper<MB, K + 2>(u.c[2], u.d[2], u.rk[2], r, v);
+  }
+  step_upper<MB, K + 1>(u.c[1], u.d[1], u.rk[1], r, v);
+  step_upper<MB, K>(u.c[0], u.d[0], u.rk[0], r, v);
+  if constexpr (S > 0) group_backward<MB, S - 1>(L, rd, r, v, next);
+}
+
+// entries of T the grouped solve keeps in LDS: the columns, 16 MB rows each,
+// zeros up to column 16 MB
+__host__ __device__ constexpr int group_entries(int mb) { return 256 * mb * mb; }
+
+// The same solve with plain divisions, the local vector in `out`: for patches
+// whose values leave divide_by's range.  16 lanes of one wavefront; a wavefront's
+// memory operations on one address are ordered once the earlier ones are waited
+// for.
+template <typename T>
+__device__ __attribute__((noinline)) void solve_plain(int m, int ld, const T* L,
+                                                      const int32_t* gi, const T* h,
+                                                      volatile T* out, int r) {
+  for (int i = r; i < m; i += 16) out[i] = h[gi[i]];
+  __builtin_amdgcn_s_waitcnt(0);
+  for (int k = 0; k < m - 1; ++k) {
+    const T y = out[k];
+    __builtin_amdgcn_s_waitcnt(0);
+    for (int i = r; i < m; i += 16)
+      if (i > k) out[i] = add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+  for (int k = m - 1; k >= 0; --k) {
+    const T y = (T)out[k] / L[k * ld + k];
+    __builtin_amdgcn_s_waitcnt(0);
+    for (int i = r; i <= k; i += 16)
+      out[i] = i == k ? y : add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+}
+
+// Patches of one class per workgroup: the factors go to LDS once (16-byte
+// loads, the first local vectors gathered meanwhile), then 16 lanes solve each
+// patch, lane r holding its rows r, r + 16, ... (MB of them), the solved value
+// broadcast to the 16 lanes by one DPP move per half.  A wavefront thus solves 4
+// patches at a time with the LDS reads shared between them; every entry sees the
+// operations of k_vanka_solve in the same order.  Bound by the chain of 2 m
+// dependent steps, not by memory: 108 unknowns, 4096 patches in 27 classes, 20.6
+// us in FP32 and 37.8 in FP64 (k_vanka_solve: 56 and 107), 512 patches 13.3 and
+// 17.2 (36 and 40).
+constexpr int kGroupThreads = 512;
+template <typename T, int MB>
+__global__ __launch_bounds__(kGroupThreads) void k_vanka_group(int m, int64_t lstride,
+                                                     const T* __restrict__ lu,
+                                                     const double* __restrict__ rdiag,
+                                                     const int32_t* __restrict__ groups,
+                                                     const int32_t* __restrict__ plist,
+                                                     const int32_t* __restrict__ gidx,
+                                                     const T* __restrict__ h,
+                                                     T* __restrict__ xp) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double rd[32 * MB];  // u_kk and its reciprocal
+  T* L = reinterpret_cast<T*>(smem);
+  const int32_t* g = groups + 3 * (int64_t)blockIdx.x;
+  const int64_t c = g[0], first = g[1];
+  const int count = g[2];
+  int r = threadIdx.x & 15;
+  int t = threadIdx.x >> 4;
+  T v[MB];
+  auto gather = [&]() {
+    const int32_t* gi = gidx + (int64_t)plist[first + t] * m;
+#pragma unroll
+    for (int j = 0; j < MB; ++j) v[j] = (16 * j + r < m) ? h[gi[16 * j + r]] : (T)0;
+  };
+  if (t < count) gather();  // in flight while the factors are staged
+  typedef int v4 __attribute__((ext_vector_type(4)));
+  constexpr int per = 16 / sizeof(T);
+  const v4* src = reinterpret_cast<const v4*>(lu + c * lstride);
+  v4* dst = reinterpret_cast<v4*>(smem);
+  const int n16 = 16 * MB * m / per, all16 = group_entries(MB) / per;
+  // up to 8 loads in flight per thread
+  for (int e0 = threadIdx.x; e0 < n16; e0 += 8 * kGroupThreads) {
+    v4 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + u * kGroupThreads;
+      x[u] = e < n16 ? src[e] : v4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + u * kGroupThreads;
+      if (e < n16) dst[e] = x[u];
+    }
+  }
+  for (int e = n16 + threadIdx.x; e < all16; e += kGroupThreads) dst[e] = v4{0, 0, 0, 0};
+  bool plain = false;  // a zero or extreme diagonal
+  for (int k = threadIdx.x; k < 16 * MB; k += kGroupThreads) {
+    rd[2 * k] = k < m ? (double)lu[c * lstride + k * (16 * MB + 1)] : 1.0;
+    rd[2 * k + 1] = k < m ? rdiag[c * m + k] : 1.0;
+    plain = rd[2 * k + 1] == 0.0;
+  }
+  plain = __syncthreads_or(plain);
+  for (; t < count;) {
+    reads_stay(r);
+    {
+      T c[kSet<T>][MB];
+      load_lower<MB, 0>(L, r, c);
+      group_forward<MB, 0>(L, r, v, c);
+    }
+    {
+      constexpr int last = 16 * MB / kSet<T> - 1;
+      UpperSet<T, MB> u;
+      load_upper<MB, last>(L, r, rd, u);
+      group_backward<MB, last>(L, rd, r, v, u);
+    }
+    const int64_t p = plist[first + t];
+    T* out = xp + p * (int64_t)m;
+    bool ok = !plain;
+#pragma unroll
+    for (int j = 0; j < MB; ++j) ok = ok && in_range(v[j]);
+    const uint64_t bad = __ballot(!ok) >> (threadIdx.x & 48);
+    if (__builtin_expect((bad & 0xFFFF) != 0, 0)) {
+      solve_plain<T>(m, 16 * MB, lu + c * lstride, gidx + p * m, h, out, r);
+    } else {
+#pragma unroll
+      for (int j = 0; j < MB; ++j)
+        if (16 * j + r < m) out[16 * j + r] = v[j];
+    }
+    t += kGroupThreads / 16;
+    if (t < count) gather();
+  }
+}
+
+// h(i, c) = (sum over the patches of node i, ascending) * (1 / count_i); mode 0
+// x = h, 1 x += omega h (StdSolver::smooth), 2 x = omega h
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_vanka_average(int64_t n, int B, int psize, int m,
                                                           const int32_t* __restrict__ nptr,
                                                           const int32_t* __restrict__ nent,
                                                           const T* __restrict__ xp,
-                                                          T* __restrict__ x) {
+                                                          T* __restrict__ x, int mode, T omega) {
   const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (t >= n * B) return;
   const int64_t i = t / B;
@@ -362,33 +708,194 @@ __global__ __launch_bounds__(kBlock) void k_vanka_average(int64_t n, int B, int 
     acc = add_rn(acc, xp[pp * m + B * r + c]);
   }
   const double s = 1.0 / (double)(e1 - e0);
-  x[t] = (T)mul_rn((double)acc, s);
+  const T h = (T)mul_rn((double)acc, s);
+  if (mode == 0)
+    x[t] = h;
+  else if (mode == 1)
+    x[t] = add_rn(x[t], mul_rn(omega, h));
+  else
+    x[t] = mul_rn(omega, h);
+}
+
+template <typename T, int MB>
+int group_launch(gh_ctx* ctx, const gh_vanka* V, const T* h) {
+  const int lds = group_entries(MB) * (int)sizeof(T);
+  hipLaunchKernelGGL((k_vanka_group<T, MB>), dim3((unsigned)V->ngroups), dim3(kGroupThreads), lds,
+                     ctx->stream, V->m, V->lstride, (const T*)V->lu, V->rdiag, V->groups, V->plist,
+                     V->piv, h, (T*)V->xp);
+  GH_HIP(hipGetLastError());
+  return GH_OK;
+}
+
+// the LDS of the grouped solve for local systems of m unknowns, allowed once
+// at creation
+template <typename T>
+bool group_allow(int m) {
+  const int mb = (m + 15) / 16;
+  const void* k[8] = {(const void*)k_vanka_group<T, 1>, (const void*)k_vanka_group<T, 2>,
+                      (const void*)k_vanka_group<T, 3>, (const void*)k_vanka_group<T, 4>,
+                      (const void*)k_vanka_group<T, 5>, (const void*)k_vanka_group<T, 6>,
+                      (const void*)k_vanka_group<T, 7>, (const void*)k_vanka_group<T, 8>};
+  return hipFuncSetAttribute(k[mb - 1], hipFuncAttributeMaxDynamicSharedMemorySize,
+                             group_entries(mb) * (int)sizeof(T)) == hipSuccess;
+}
+
+template <typename T>
+int vanka_apply_t(gh_ctx* ctx, const gh_vanka* V, const T* in, T* out, int mode, T omega) {
+  if (V->ngroups > 0) {
+    int rc = GH_OK;
+    switch ((V->m + 15) / 16) {
+      case 1: rc = group_launch<T, 1>(ctx, V, in); break;
+      case 2: rc = group_launch<T, 2>(ctx, V, in); break;
+      case 3: rc = group_launch<T, 3>(ctx, V, in); break;
+      case 4: rc = group_launch<T, 4>(ctx, V, in); break;
+      case 5: rc = group_launch<T, 5>(ctx, V, in); break;
+      case 6: rc = group_launch<T, 6>(ctx, V, in); break;
+      case 7: rc = group_launch<T, 7>(ctx, V, in); break;
+      default: rc = group_launch<T, 8>(ctx, V, in); break;
+    }
+    GH_TRY(rc);
+  } else {
+    const unsigned gs = (unsigned)((V->npatches + kBlock / 64 - 1) / (kBlock / 64));
+    hipLaunchKernelGGL(k_vanka_solve<T>, dim3(gs), dim3(kBlock), 0, ctx->stream, V->npatches,
+                       V->psize, V->B, V->cls, V->ld, (const T*)V->lu, V->piv, in, (T*)V->xp);
+  }
+  const unsigned ga = (unsigned)((V->n * V->B + kBlock - 1) / kBlock);
+  hipLaunchKernelGGL(k_vanka_average<T>, dim3(ga), dim3(kBlock), 0, ctx->stream, V->n, V->B,
+                     V->psize, V->m, V->nptr, V->nent, (const T*)V->xp, out, mode, omega);
+  GH_HIP(hipGetLastError());
+  return GH_OK;
+}
+
+// The patches by class: cls[p], and reps[c] the first patch of class c (classes
+// in order of first appearance).  Patches whose hashes agree but whose entries
+// do not each get a class of their own.
+int patch_classes(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, int B,
+                  const int32_t* d_nodes, std::vector<int32_t>& cls, std::vector<int32_t>& reps) {
+  const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
+  uint64_t* d_hash = nullptr;
+  int32_t* d_rep = nullptr;
+  std::vector<uint64_t> hash(2 * npatches);
+  std::vector<int32_t> first(npatches), differs(npatches, 0);
+  int rc = GH_OK;
+  auto run = [&]() -> int {
+    if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * 2 * npatches) != hipSuccess ||
+        hipMalloc((void**)&d_rep, sizeof(int32_t) * 2 * npatches) != hipSuccess)
+      return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
+    GH_HIP(hipFuncSetAttribute((const void*)k_vanka_hash,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    GH_HIP(hipFuncSetAttribute((const void*)k_vanka_same,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * lds)));
+    hipLaunchKernelGGL(k_vanka_hash, dim3((unsigned)npatches), dim3(kHashThreads), lds,
+                       ctx->stream, psize, B, d_nodes, A->rowptr, A->col, (const double*)A->val,
+                       d_hash);
+    GH_HIP(hipGetLastError());
+    GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * hash.size(),
+                          hipMemcpyDeviceToHost, ctx->stream));
+    GH_HIP(hipStreamSynchronize(ctx->stream));
+    bool shared = false;
+    {
+      // both sums must agree; the first patch with a pair stands for it
+      std::vector<int32_t> by(npatches);
+      for (int64_t p = 0; p < npatches; ++p) by[p] = (int32_t)p;
+      std::sort(by.begin(), by.end(), [&](int32_t a, int32_t b) {
+        if (hash[2 * a] != hash[2 * b]) return hash[2 * a] < hash[2 * b];
+        if (hash[2 * a + 1] != hash[2 * b + 1]) return hash[2 * a + 1] < hash[2 * b + 1];
+        return a < b;
+      });
+      int32_t f = npatches > 0 ? by[0] : 0;
+      for (int64_t i = 0; i < npatches; ++i) {
+        const int32_t p = by[i];
+        if (hash[2 * p] != hash[2 * f] || hash[2 * p + 1] != hash[2 * f + 1]) f = p;
+        first[p] = f;
+        shared = shared || f != p;
+      }
+    }
+    if (shared) {
+      GH_HIP(hipMemcpyAsync(d_rep, first.data(), sizeof(int32_t) * npatches, hipMemcpyHostToDevice,
+                            ctx->stream));
+      GH_HIP(hipMemcpyAsync(d_rep + npatches, differs.data(), sizeof(int32_t) * npatches,
+                            hipMemcpyHostToDevice, ctx->stream));
+      hipLaunchKernelGGL(k_vanka_same, dim3((unsigned)npatches), dim3(kHashThreads), 2 * lds,
+                         ctx->stream, psize, B, d_nodes, A->rowptr, A->col,
+                         (const double*)A->val, d_rep, d_rep + npatches);
+      GH_HIP(hipGetLastError());
+      GH_HIP(hipMemcpyAsync(differs.data(), d_rep + npatches, sizeof(int32_t) * npatches,
+                            hipMemcpyDeviceToHost, ctx->stream));
+      GH_HIP(hipStreamSynchronize(ctx->stream));
+    }
+    return GH_OK;
+  };
+  rc = run();
+  if (d_hash) (void)hipFree(d_hash);
+  if (d_rep) (void)hipFree(d_rep);
+  GH_TRY(rc);
+  cls.assign(npatches, -1);
+  reps.clear();
+  for (int64_t p = 0; p < npatches; ++p) {  // first[p] <= p
+    if (first[p] == p || differs[p]) {
+      cls[p] = (int32_t)reps.size();
+      reps.push_back((int32_t)p);
+    } else {
+      cls[p] = cls[first[p]];
+    }
+  }
+  return GH_OK;
+}
+
+// Whether the grouped solve runs, and its groups.
+int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
+  const int64_t np = V->npatches, nc = V->nclasses;
+  const int mb = (V->m + 15) / 16;
+  const int64_t ts = V->prec == GH_F64 ? 8 : 4;
+  const int64_t lds = group_entries(mb) * ts + 256 * mb;
+  const int64_t fit = std::min<int64_t>(8, (160 << 10) / lds);  // workgroups a CU holds
+  const int64_t at_once = fit * ctx->num_cu;
+  // Distinct factors are read once either way: the grouped solve is faster while
+  // every patch has a workgroup at once (216 patches of 108 unknowns 16 us
+  // against 36 in FP32, 1728 patches 69 against 42), shared factors always.
+  if (np < 2 * nc && np > at_once) return GH_OK;
+  if (!(V->prec == GH_F64 ? group_allow<double>(V->m) : group_allow<float>(V->m))) {
+    (void)hipGetLastError();
+    return GH_OK;
+  }
+  // a wavefront takes 4 patches at a time: as many per workgroup as fill the
+  // chip once, over 8 wavefronts
+  const int64_t chunk = 4 * std::max<int64_t>(1, (np + 4 * at_once - 1) / (4 * at_once));
+  std::vector<int64_t> start(nc + 1, 0);
+  for (int64_t p = 0; p < np; ++p) start[cls[p] + 1]++;
+  for (int64_t c = 0; c < nc; ++c) start[c + 1] += start[c];
+  std::vector<int32_t> plist(np), groups;
+  {
+    std::vector<int64_t> fill(start.begin(), start.end() - 1);
+    for (int64_t p = 0; p < np; ++p) plist[fill[cls[p]]++] = (int32_t)p;
+  }
+  for (int64_t c = 0; c < nc; ++c)
+    for (int64_t a = start[c]; a < start[c + 1]; a += chunk) {
+      groups.push_back((int32_t)c);
+      groups.push_back((int32_t)a);
+      groups.push_back((int32_t)std::min(chunk, start[c + 1] - a));
+    }
+  if (hipMalloc((void**)&V->plist, sizeof(int32_t) * np) != hipSuccess ||
+      hipMalloc((void**)&V->groups, sizeof(int32_t) * groups.size()) != hipSuccess)
+    return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
+  GH_HIP(hipMemcpy(V->plist, plist.data(), sizeof(int32_t) * np, hipMemcpyHostToDevice));
+  GH_HIP(hipMemcpy(V->groups, groups.data(), sizeof(int32_t) * groups.size(), hipMemcpyHostToDevice));
+  V->ngroups = (int64_t)groups.size() / 3;
+  return GH_OK;
 }
 
 }  // namespace
 
 namespace gh {
 
-int vanka_solve(gh_ctx* ctx, const gh_vanka* V, int prec, void* x) {
+int vanka_apply(gh_ctx* ctx, const gh_vanka* V, int prec, const void* in, void* out, int mode,
+                double omega) {
   if (prec != V->prec) return fail(GH_EINVAL, "vanka: vector precision differs from the factors'");
-  const unsigned gs = (unsigned)((V->npatches + kBlock / 64 - 1) / (kBlock / 64));
-  const unsigned ga = (unsigned)((V->n * V->B + kBlock - 1) / kBlock);
   if (V->npatches == 0) return GH_OK;
-  if (prec == GH_F64) {
-    hipLaunchKernelGGL(k_vanka_solve<double>, dim3(gs), dim3(kBlock), 0, ctx->stream, V->npatches,
-                       V->psize, V->B, (const double*)V->lu, V->piv, (const double*)x,
-                       (double*)V->xp);
-    hipLaunchKernelGGL(k_vanka_average<double>, dim3(ga), dim3(kBlock), 0, ctx->stream, V->n, V->B,
-                       V->psize, V->m, V->nptr, V->nent, (const double*)V->xp, (double*)x);
-  } else {
-    hipLaunchKernelGGL(k_vanka_solve<float>, dim3(gs), dim3(kBlock), 0, ctx->stream, V->npatches,
-                       V->psize, V->B, (const float*)V->lu, V->piv, (const float*)x,
-                       (float*)V->xp);
-    hipLaunchKernelGGL(k_vanka_average<float>, dim3(ga), dim3(kBlock), 0, ctx->stream, V->n, V->B,
-                       V->psize, V->m, V->nptr, V->nent, (const float*)V->xp, (float*)x);
-  }
-  GH_HIP(hipGetLastError());
-  return GH_OK;
+  if (prec == GH_F64)
+    return vanka_apply_t<double>(ctx, V, (const double*)in, (double*)out, mode, omega);
+  return vanka_apply_t<float>(ctx, V, (const float*)in, (float*)out, mode, (float)omega);
 }
 
 int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, const int32_t* nodes,
@@ -440,7 +947,8 @@ int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, cons
     return hipMalloc(p, std::max<size_t>(bytes, 8)) == hipSuccess;
   };
   if (!alloc((void**)&V->nodes, sizeof(int32_t) * npatches * psize) ||
-      !alloc(&V->lu, ts * npatches * m * m) || !alloc((void**)&V->piv, sizeof(int32_t) * npatches * m) ||
+      !alloc((void**)&V->cls, sizeof(int32_t) * npatches) ||
+      !alloc((void**)&V->piv, sizeof(int32_t) * npatches * m) ||
       !alloc((void**)&V->nptr, sizeof(int32_t) * (n + 1)) ||
       !alloc((void**)&V->nent, sizeof(int32_t) * npatches * psize) ||
       !alloc(&V->xp, ts * npatches * m))
@@ -450,36 +958,71 @@ int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, cons
       hipMemcpy(V->nent, nent.data(), sizeof(int32_t) * npatches * psize, hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(GH_EHIP, "gh_vanka_create: upload failed"));
   if (npatches > 0) {
-    const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
-    if (hipFuncSetAttribute((const void*)k_vanka_factor, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess)
-      return bail(fail(GH_EHIP, "gh_vanka_create: %zu bytes of LDS per patch not available", lds));
-    hipLaunchKernelGGL(k_vanka_factor, dim3((unsigned)npatches), dim3(kFactorThreads), lds,
-                       ctx->stream,
-                       npatches, psize, B, V->nodes, A->rowptr, A->col, (const double*)A->val,
-                       prec == GH_F64 ? (double*)V->lu : nullptr,
-                       prec == GH_F64 ? nullptr : (float*)V->lu, V->piv);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess)
-      return bail(fail(GH_EHIP, "gh_vanka_create: factorisation failed"));
+    std::vector<int32_t> cls, reps;
+    if (int rc = patch_classes(ctx, A, npatches, psize, B, V->nodes, cls, reps)) return bail(rc);
+    const int64_t nc = V->nclasses = (int64_t)reps.size();
+    V->ld = (m + 15) / 16 * 16;
+    V->lstride = (int64_t)V->ld * m;
+    int32_t* d_reps = nullptr;
+    auto factor = [&](std::vector<int32_t>& piv) -> int {
+      if (!alloc(&V->lu, ts * nc * V->lstride) || !alloc((void**)&V->rdiag, sizeof(double) * nc * m) ||
+          !alloc((void**)&d_reps, sizeof(int32_t) * nc * (1 + m)))
+        return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
+      int32_t* d_piv = d_reps + nc;
+      GH_HIP(hipMemcpyAsync(d_reps, reps.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice,
+                            ctx->stream));
+      GH_HIP(hipMemcpyAsync(V->cls, cls.data(), sizeof(int32_t) * npatches, hipMemcpyHostToDevice,
+                            ctx->stream));
+      GH_HIP(hipMemsetAsync(V->lu, 0, ts * nc * V->lstride, ctx->stream));
+      const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
+      GH_HIP(hipFuncSetAttribute((const void*)k_vanka_factor,
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      hipLaunchKernelGGL(k_vanka_factor, dim3((unsigned)nc), dim3(kFactorThreads), lds, ctx->stream,
+                         psize, B, d_reps, V->nodes, A->rowptr, A->col, (const double*)A->val,
+                         V->ld, prec == GH_F64 ? (double*)V->lu : nullptr,
+                         prec == GH_F64 ? nullptr : (float*)V->lu, d_piv);
+      GH_HIP(hipGetLastError());
+      const dim3 gr((unsigned)((nc * m + kBlock - 1) / kBlock));
+      if (prec == GH_F64)
+        hipLaunchKernelGGL(k_vanka_rdiag<double>, gr, dim3(kBlock), 0, ctx->stream, nc, m,
+                           V->ld, (const double*)V->lu, V->rdiag);
+      else
+        hipLaunchKernelGGL(k_vanka_rdiag<float>, gr, dim3(kBlock), 0, ctx->stream, nc, m,
+                           V->ld, (const float*)V->lu, V->rdiag);
+      GH_HIP(hipGetLastError());
+      piv.resize((size_t)nc * m);
+      GH_HIP(hipMemcpyAsync(piv.data(), d_piv, sizeof(int32_t) * piv.size(), hipMemcpyDeviceToHost,
+                            ctx->stream));
+      GH_HIP(hipStreamSynchronize(ctx->stream));
+      return GH_OK;
+    };
+    std::vector<int32_t> piv;
+    const int frc = factor(piv);
+    if (d_reps) (void)hipFree(d_reps);
+    if (frc) return bail(frc);
     // Compose the recorded row exchanges (applied in order k = 0..m-1) into
     // one gather: row i of P h is local entry src[i], i.e. the global entry
     // node(src[i] / B) * B + src[i] % B.  The solve then needs no exchanges.
-    std::vector<int32_t> piv((size_t)npatches * m);
-    if (hipMemcpy(piv.data(), V->piv, sizeof(int32_t) * piv.size(), hipMemcpyDeviceToHost) != hipSuccess)
-      return bail(fail(GH_EHIP, "gh_vanka_create: pivot download failed"));
-    std::vector<int32_t> src(m);
-    for (int64_t p = 0; p < npatches; ++p) {
-      int32_t* pv = piv.data() + p * m;
-      for (int i = 0; i < m; ++i) src[i] = i;
+    std::vector<int32_t> src((size_t)nc * m), gidx((size_t)npatches * m);
+    for (int64_t c = 0; c < nc; ++c) {
+      const int32_t* pv = piv.data() + c * m;
+      int32_t* sc = src.data() + c * m;
+      for (int i = 0; i < m; ++i) sc[i] = i;
       for (int k = 0; k < m; ++k) {
         if (pv[k] < k || pv[k] >= m) return bail(fail(GH_EINVAL, "gh_vanka_create: bad pivot"));
-        std::swap(src[k], src[pv[k]]);
+        std::swap(sc[k], sc[pv[k]]);
       }
-      for (int i = 0; i < m; ++i)
-        pv[i] = (int32_t)((int64_t)nodes[p * psize + src[i] / B] * B + src[i] % B);
     }
-    if (hipMemcpy(V->piv, piv.data(), sizeof(int32_t) * piv.size(), hipMemcpyHostToDevice) != hipSuccess)
+    parallel_for(npatches, 2048, [&](int64_t a, int64_t b) {
+      for (int64_t p = a; p < b; ++p) {
+        const int32_t* sc = src.data() + (int64_t)cls[p] * m;
+        for (int i = 0; i < m; ++i)
+          gidx[p * m + i] = (int32_t)((int64_t)nodes[p * psize + sc[i] / B] * B + sc[i] % B);
+      }
+    });
+    if (hipMemcpy(V->piv, gidx.data(), sizeof(int32_t) * gidx.size(), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(GH_EHIP, "gh_vanka_create: gather upload failed"));
+    if (int rc = vanka_groups(ctx, V, cls)) return bail(rc);
   }
   *out = V;
   return GH_OK;
@@ -499,7 +1042,8 @@ int gh_vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize,
 int gh_vanka_destroy(gh_vanka* V) {
   if (!V) return GH_OK;
   if (V->ctx && V->ctx->stream) (void)hipStreamSynchronize(V->ctx->stream);
-  for (void* p : {(void*)V->nodes, V->lu, (void*)V->piv, (void*)V->nptr, (void*)V->nent, V->xp})
+  for (void* p : {(void*)V->nodes, (void*)V->cls, V->lu, (void*)V->rdiag, (void*)V->piv,
+                  (void*)V->nptr, (void*)V->nent, V->xp, (void*)V->groups, (void*)V->plist})
     if (p) (void)hipFree(p);
   gh_ctx* ctx = V->ctx;
   delete V;
@@ -510,7 +1054,7 @@ int gh_vanka_destroy(gh_vanka* V) {
 int gh_vanka_solve(gh_ctx* ctx, const gh_vanka* V, gh_vec* x) {
   GH_ARG(ctx && V && x, "gh_vanka_solve: NULL argument");
   GH_ARG(x->n == V->n && x->ncomp == V->B, "gh_vanka_solve: vector shape does not match");
-  return vanka_solve(ctx, V, x->prec, x->d);
+  return vanka_apply(ctx, V, x->prec, x->d, x->d, 0, 1.0);
 }
 
 }  // extern "C"

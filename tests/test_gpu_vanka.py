@@ -108,3 +108,54 @@ def test_vanka_mixed_precision_solve(ctx):
                    H.NLInfo(1e-10, 1e-30, 30), norm_kind=1)
     assert H.N.NL_STATUS[rep.status] == "converged"
     assert np.linalg.norm(U.copy_back() - uo) <= 1e-8 * np.linalg.norm(uo)
+
+
+def plane_problem(refine, B, seed, vary, children=4):
+    """a 2D hierarchy's finest level with a B-component block operator, patches of
+    9 nodes (4 cells) or 25 (16 cells); `vary`: a coefficient per cell, so that no two patches are equal"""
+    M = Mesh("square.inp", 2, refine, 1)
+    r = np.random.default_rng(seed)
+    k = r.uniform(0.5, 2.0, len(M.cells(M.nlevels - 1))) if vary else None
+    lev = assemble_hierarchy(M, k).fine
+    C = np.eye(B) + 0.2 * r.uniform(-1, 1, (B, B))
+    val = lev.val if B == 1 else block_operator(lev, C, 0.1 * r.uniform(-1, 1, (B, B)))
+    return lev, np.asarray(val), patches_from_cells(M.cells(M.nlevels - 1), children), r
+
+
+# local systems of 9 .. 125 unknowns (1 to 8 rows per lane, full and partial),
+# patches that share factors and patches that do not, and more distinct patches
+# than the grouped solve takes (16,384: one wavefront per patch)
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("B,refine,vary,children",
+                         [(1, 2, True, 4), (1, 4, False, 4), (2, 4, True, 4), (4, 3, False, 4),
+                          (5, 3, True, 4), (7, 3, True, 4), (8, 2, True, 4), (3, 4, True, 16),
+                          (4, 4, False, 16), (5, 4, True, 16), (1, 8, True, 4)])
+def test_vanka_solve_shapes(ctx, prec, B, refine, vary, children):
+    print(f"[vanka B={B} refine={refine} vary={vary} {children} {prec}]", flush=True)
+    lev, val, pat, r = plane_problem(refine, B, 100 * B + refine, vary, children)
+    x = r.uniform(-1, 1, lev.n * B)
+    A = H.CudaCSRMatrixInterface(ctx, lev.rowptr, lev.col, val, B)
+    X = H.CudaVectorInterface.from_global(ctx, x, B, prec)
+    H.VankaSmoother(ctx, A, pat, prec).solve(X)
+    xo = x.copy()
+    O.Vanka(O.Matrix(lev.rowptr, lev.col, val, B), pat).solve(xo)
+    if prec == "f64":
+        assert np.array_equal(X.copy_back(), xo)
+    else:
+        assert np.abs(X.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
+
+
+# factors and vectors outside the range in which the grouped solve multiplies by
+# reciprocals: those patches are solved with plain divisions
+@pytest.mark.parametrize("ascale,xscale", [(2.0 ** 500, 1.0), (2.0 ** -450, 2.0 ** -300),
+                                           (1.0, 2.0 ** -800), (1.0, 2.0 ** 700)])
+def test_vanka_solve_extreme_values(ctx, ascale, xscale):
+    lev, val, pat, r = plane_problem(3, 2, 5, True)
+    val = val * ascale
+    x = r.uniform(-1, 1, lev.n * 2) * xscale
+    x[::3] = 0.0
+    X = H.CudaVectorInterface.from_global(ctx, x, 2)
+    H.VankaSmoother(ctx, H.CudaCSRMatrixInterface(ctx, lev.rowptr, lev.col, val, 2), pat).solve(X)
+    xo = x.copy()
+    O.Vanka(O.Matrix(lev.rowptr, lev.col, val, 2), pat).solve(xo)
+    assert np.array_equal(X.copy_back(), xo)
