@@ -308,18 +308,21 @@ int vec_fill_zero(gh_ctx* ctx, int prec, int64_t size, void* x) {
 
 // ------------------------------------------------------------------ SpMV
 // block matrices (ncomp > 1): one thread per block row component
+template <int B, typename VT, typename XT, typename Acc, class Op>
+static void launch_bsell_as(gh_ctx* ctx, const BSell& S, const XT* x, Op op) {
+  hipLaunchKernelGGL((k_bsell<B, VT, XT, Acc, Op>), dim3((unsigned)S.nslices),
+                     dim3(64 * kBSplit), 0, ctx->stream, S.sptr, S.row, S.rlen, S.col,
+                     (const VT*)S.val, x, op);
+}
+
 template <int B, typename XT, typename Acc, class Op>
 static void launch_bsell(gh_ctx* ctx, const BSell& S, const XT* x, Op op) {
-  const unsigned grid = grid_for(S.nslices * 64);
   if (S.prec == GH_F64)
-    hipLaunchKernelGGL((k_bsell<B, double, XT, Acc, Op>), dim3(grid), dim3(kBlock), 0, ctx->stream,
-                       S.nslices, S.sptr, S.row, S.rlen, S.col, (const double*)S.val, x, op);
+    launch_bsell_as<B, double, XT, Acc>(ctx, S, x, op);
   else if (S.prec == GH_F32)
-    hipLaunchKernelGGL((k_bsell<B, float, XT, Acc, Op>), dim3(grid), dim3(kBlock), 0, ctx->stream,
-                       S.nslices, S.sptr, S.row, S.rlen, S.col, (const float*)S.val, x, op);
+    launch_bsell_as<B, float, XT, Acc>(ctx, S, x, op);
   else
-    hipLaunchKernelGGL((k_bsell<B, __half, XT, Acc, Op>), dim3(grid), dim3(kBlock), 0, ctx->stream,
-                       S.nslices, S.sptr, S.row, S.rlen, S.col, (const __half*)S.val, x, op);
+    launch_bsell_as<B, __half, XT, Acc>(ctx, S, x, op);
 }
 
 template <typename XT, typename Acc, class Op>
