@@ -40,6 +40,9 @@ struct SpmvOp {  // y = d * (A x) + b * y
   bool read_y;
   __device__ __forceinline__ T init(int64_t) const { return (T)0; }
   __device__ __forceinline__ T step(T acc, T a, T x) const { return fma_step<T, EXACT>(acc, a, x); }
+  // the step of a product formed and rounded before (exact ops)
+  __device__ __forceinline__ T fold(T acc, T p) const { return add_rn(acc, p); }
+  static __device__ __forceinline__ T neutral() { return (T)-0.0; }  // fold(acc, neutral) = acc
   __device__ __forceinline__ void finish(int64_t r, T acc) const {
     T v = EXACT ? mul_rn(d, acc) : d * acc;
     if (read_y) v = EXACT ? add_rn(v, mul_rn(b, (T)y[r])) : v + b * (T)y[r];
@@ -54,6 +57,8 @@ struct ResidualOp {  // r = b - A x: r starts at b and subtracts each a_ij x_j i
   const T* b;
   __device__ __forceinline__ T init(int64_t i) const { return b[i]; }
   __device__ __forceinline__ T step(T acc, T a, T x) const { return fms_step<T, EXACT>(acc, a, x); }
+  __device__ __forceinline__ T fold(T acc, T p) const { return add_rn(acc, -p); }
+  static __device__ __forceinline__ T neutral() { return (T)0.0; }
   __device__ __forceinline__ void finish(int64_t i, T acc) const { r[i] = acc; }
 };
 
@@ -68,6 +73,8 @@ struct JacobiOp {  // xn = x + omega * (dinv * (b - A x))
   int richardson;
   __device__ __forceinline__ T init(int64_t i) const { return b[i]; }
   __device__ __forceinline__ T step(T acc, T a, T xx) const { return fms_step<T, EXACT>(acc, a, xx); }
+  __device__ __forceinline__ T fold(T acc, T p) const { return add_rn(acc, -p); }
+  static __device__ __forceinline__ T neutral() { return (T)0.0; }
   __device__ __forceinline__ void finish(int64_t i, T h) const {
     if (!richardson) h = EXACT ? mul_rn((T)dinv[i], h) : (T)dinv[i] * h;
     xn[i] = EXACT ? add_rn(x[i], mul_rn(omega, h)) : x[i] + omega * h;
@@ -414,6 +421,119 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_split(
   }
 }
 
+// k_sell for exact ops on long rows, whose chains of loads and scattered gathers
+// (caller's entry order) bound one wavefront per slice: a workgroup of K wavefronts
+// per slice forms the rounded products of K * E entries of the 64 rows at a time,
+// side by side, into LDS, and wavefront 0 folds them into the rows in entry
+// order -- the additions of k_sell in the same order, bit for bit.  Entry k of a
+// round goes to wavefront k % K.  Entries past the slice's width repeat its last
+// one (their values and columns exist), and every product past a row's end is
+// replaced by the fold's neutral element.  The loads run ahead of the fold: while
+// a round is folded the next one's values and x entries and the columns after
+// that are in flight.  Two buffers, one barrier per round.
+template <typename VT, typename XT, typename T, class Op, int K>
+__global__ __launch_bounds__(kSlice * K) void k_sell_fold(
+    int64_t n, const uint32_t* __restrict__ sptr, const uint16_t* __restrict__ rlen,
+    const uint16_t* __restrict__ cidx, const uint32_t* __restrict__ cptr,
+    const uint32_t* __restrict__ cbase, const int32_t* __restrict__ ptab,
+    const int32_t* __restrict__ pstart, const VT* __restrict__ val,
+    const int32_t* __restrict__ perm, const XT* __restrict__ x, Op op) {
+  constexpr int E = 8, C = K * E;
+  __shared__ T part[2][C][kSlice];
+  const int64_t s = xcd_block(blockIdx.x, gridDim.x);  // one slice per workgroup
+  const int lane = threadIdx.x & (kSlice - 1);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kSlice));
+  const int64_t slot0 = s * kSlice + lane;
+  const bool active = slot0 < n;
+  const int64_t slot = active ? slot0 : n - 1;
+  const int64_t row = perm ? (int64_t)perm[slot] : slot;
+  const uint32_t v0 = sptr[s];
+  const int width = (int)((sptr[s + 1] - v0) / kSlice);
+  const VT* vp = val + v0 + lane;
+  const uint32_t meta = cptr[s];
+  const uint32_t cb = cbase[s];
+  const bool patterned = (meta & 0x40000000u) != 0, wide = (meta & 0x80000000u) != 0;
+  int len = 0;
+  const int32_t* off = ptab;
+  if (patterned) {
+    const int pid = (meta & 0x20000000u) ? __builtin_amdgcn_readfirstlane((int)cb) : (int)rlen[slot];
+    const int p0 = pstart[pid];
+    off = ptab + p0;
+    len = pstart[pid + 1] - p0;
+  } else {
+    len = rlen[slot];
+  }
+  const uint16_t* c16 = cidx + (meta & 0x1FFFFFFFu) + lane;
+  const uint32_t* c32 = (const uint32_t*)(cidx + (meta & 0x1FFFFFFFu)) + lane;
+  uint32_t c[E];
+  T a[E], xv[E];
+  auto columns = [&](int c0) {
+    if (patterned) {
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        const int k = c0 + u * K + w;
+        c[u] = (uint32_t)row + (k < len ? off[k] : 0);
+      }
+    } else if (wide) {
+#pragma unroll
+      for (int u = 0; u < E; ++u) c[u] = c32[(int64_t)min(c0 + u * K + w, width - 1) * kSlice];
+    } else {
+#pragma unroll
+      for (int u = 0; u < E; ++u)
+        c[u] = cb + c16[(int64_t)min(c0 + u * K + w, width - 1) * kSlice];
+    }
+  };
+  auto entries = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) a[u] = (T)ld(vp + (int64_t)min(c0 + u * K + w, width - 1) * kSlice);
+#pragma unroll
+    for (int u = 0; u < E; ++u) xv[u] = (T)x[c[u]];
+  };
+  T acc = (T)0;
+  if (w == 0) acc = op.init(row);
+  if (width > 0) {
+    columns(0);
+    entries(0);
+    if (C < width) columns(C);
+  }
+  for (int c0 = 0, buf = 0; c0 < width; c0 += C, buf ^= 1) {
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      part[buf][u * K + w][lane] = c0 + u * K + w < len ? mul_rn(a[u], xv[u]) : Op::neutral();
+    __syncthreads();
+    if (c0 + C < width) entries(c0 + C);
+    if (c0 + 2 * C < width) columns(c0 + 2 * C);
+    __builtin_amdgcn_sched_barrier(0);
+    if (w == 0) {
+#pragma unroll
+      for (int u0 = 0; u0 < C; u0 += 16) {
+        if (c0 + u0 < width) {
+          T q[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) q[u] = part[buf][u0 + u][lane];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) acc = op.fold(acc, q[u]);
+        }
+      }
+    }
+  }
+  if (w == 0 && active) op.finish(row, acc);
+}
+
+// Wavefronts per slice of an exact sweep (0: k_sell).  The fold pays where rows
+// are long; rows of up to 27 entries (Q1) are faster in k_sell from 117 K rows up
+// (7.8 against 10.1 us) and equal below.  Two rounds of 64 entries keep few
+// slices busier than four of 32, which leave LDS for more slices per CU: FP64
+// residuals of Q2 rows (62 entries on average, 125 to 285 at most), k_sell / 4 / 8
+// wavefronts: 729 rows 8.3 / 6.7 / 5.4 us, 14 K 17.5 / 11.7 / 9.0, 79 K 38 / 27 /
+// 24, 275 K 60 / 45 / 56, 352 K 109 / 64 / 78.
+constexpr int kFoldRow = 32;
+constexpr int64_t kFoldFewSlices = 2048;
+inline int sell_fold_waves(const Sell& S) {
+  if (S.maxlen <= kFoldRow) return 0;
+  return S.nslices <= kFoldFewSlices ? 8 : 4;
+}
+
 // Split factor of a reduced-precision sweep: double K while the level runs
 // fewer than 8192 wavefronts (32 per CU) and every wavefront still gets at
 // least 8 of the longest row's entries, up to 16 wavefronts per slice.
@@ -521,6 +641,15 @@ inline int sell_w_split_launch(gh_ctx* ctx, const Sell& S, const T* x, Op op) {
 }
 
 template <typename VT, typename XT, typename T, class Op, int K>
+inline int sell_fold_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
+  hipLaunchKernelGGL((k_sell_fold<VT, XT, T, Op, K>), dim3((unsigned)S.nslices), dim3(kSlice * K),
+                     0, ctx->stream, S.n, S.sptr, S.rlen, S.cidx, S.cptr, S.cbase, S.ptab,
+                     S.pstart, (const VT*)S.val, S.perm, x, op);
+  GH_HIP(hipGetLastError());
+  return GH_OK;
+}
+
+template <typename VT, typename XT, typename T, class Op, int K>
 inline int sell_split_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
   hipLaunchKernelGGL((k_sell_split<VT, XT, T, Op, K>), dim3((unsigned)S.nslices),
                      dim3(kSlice * K), 0, ctx->stream, S.n, S.sptr, S.rlen, S.cidx, S.cptr,
@@ -538,6 +667,12 @@ inline int sell_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
       case 4: return sell_split_launch<VT, XT, T, Op, 4>(ctx, S, x, op);
       case 8: return sell_split_launch<VT, XT, T, Op, 8>(ctx, S, x, op);
       case 16: return sell_split_launch<VT, XT, T, Op, 16>(ctx, S, x, op);
+      default: break;
+    }
+  } else {
+    switch (sell_fold_waves(S)) {
+      case 4: return sell_fold_launch<VT, XT, T, Op, 4>(ctx, S, x, op);
+      case 8: return sell_fold_launch<VT, XT, T, Op, 8>(ctx, S, x, op);
       default: break;
     }
   }

@@ -572,6 +572,19 @@ def test_reduced_precision_sweeps_long_rows(ctx, n, L, prec):
         assert np.all(np.abs(X.copy_back() - want) <= bound), smoother
 
 
+@pytest.mark.parametrize("n,L", [(90, 33), (700, 40), (5000, 64), (700, 66), (5000, 100), (90, 128),
+                                 (700, 130), (700, 300), (70000, 50), (132000, 36)])
+def test_fp64_sweeps_long_rows_bitexact(ctx, n, L):
+    """Rows longer than the 32 entries from which FP64 sweeps form their
+    products on 4 or 8 wavefronts per slice and fold them in entry order:
+    around the rounds of 32 and 64 entries, partial last slices, every column
+    encoding, 8 wavefronts (up to 2048 slices) and 4: the oracle's bits."""
+    print(f"[n={n} L={L}]", flush=True)
+    rowptr, col, val = long_row_matrix(n, L, seed=3 * L + n)
+    A = H.CudaCSRMatrixInterface(ctx, rowptr, col, val)
+    check_products_vs_oracle(ctx, A, rowptr, col, val, L)
+
+
 @pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
 @pytest.mark.parametrize("name", ["q1_2d_128", "q1_3d_16", "q1_3d_8_ada", "q2_3d_8_ada"])
 def test_flexible_gmres_solve(ctx, name, prec):
