@@ -121,6 +121,41 @@ def test_block_ilu_random_order(ctx, B):
     assert np.abs(X32.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
 
 
+def banded(n, offsets, seed):
+    """a diagonally dominant matrix with entries at +-offsets from the diagonal"""
+    r = np.random.default_rng(seed)
+    off = np.unique(np.concatenate([[0], offsets, -np.asarray(offsets)]))
+    c = np.arange(n)[:, None] + off[None]
+    keep = (c >= 0) & (c < n)
+    rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    v = r.uniform(-1, 1, c.shape)
+    v[:, off == 0] = len(off) + 1.0
+    return rp, c[keep].astype(np.int32), v[keep]
+
+
+# rows of up to 90 entries per triangle (three rounds of 32 in the folded
+# sweeps), and a red-black order whose levels (2344 slices) run one wavefront
+# per slice
+@pytest.mark.parametrize("n,offsets,order", [(700, range(1, 91), None), (5000, (1, 70, 71, 4000), "random"),
+                                             (300_001, (1,), "redblack")])
+def test_scalar_ilu_shapes(ctx, n, offsets, order):
+    print(f"[ilu n={n} {order}]", flush=True)
+    rp, col, val = banded(n, list(offsets), n)
+    perm = {None: None, "random": np.random.default_rng(2).permutation(n).astype(np.int32),
+            "redblack": np.concatenate([np.arange(0, n, 2), np.arange(1, n, 2)]).astype(np.int32)}[order]
+    I = H.SparseBlockIlu(ctx, H.CudaCSRMatrixInterface(ctx, rp, col, val), perm)
+    Io = O.Ilu(O.Matrix(rp, col, val), perm)
+    x = np.random.default_rng(9).uniform(-1, 1, n)
+    X = H.CudaVectorInterface.from_global(ctx, x)
+    I.solve(X)
+    xo = x.copy()
+    Io.solve(xo)
+    assert np.array_equal(X.copy_back(), xo)
+    X32 = H.CudaVectorInterface.from_global(ctx, x, 1, "f32")
+    I.solve(X32)
+    assert np.abs(X32.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
+
+
 def test_colour_order_levels_and_solve(ctx):
     """in the colour order each triangle has one level per colour; factors and
     solves still equal the oracle's, and the FP32 solve is close"""
