@@ -198,6 +198,9 @@ struct gh_ctx {
   // rocBLAS handle on `stream` for the direct coarse factorisation (created
   // on first use, destroyed with the context)
   void* blas = nullptr;
+  // workspace of the direct coarse inverse (grown on use, freed with the context)
+  void* direct_ws = nullptr;
+  size_t direct_bytes = 0;
 };
 
 struct gh_vec {

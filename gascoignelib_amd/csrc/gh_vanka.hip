@@ -38,52 +38,6 @@ constexpr int kFactorWaves = kFactorThreads / kFactorLanes;  // columns tc + 16 
 constexpr int kRowsPer = kVankaMaxM / kFactorLanes;       // 2
 constexpr int kColsPer = kVankaMaxM / kFactorWaves;       // 8
 
-// DPP move of a double (both halves); lanes the masks leave out read 0.
-template <int CTRL, int ROWMASK, int BANKMASK>
-__device__ __forceinline__ double dpp_move(double x) {
-  const int64_t b = __builtin_bit_cast(int64_t, x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xFFFFFFFF), CTRL, ROWMASK, BANKMASK, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWMASK, BANKMASK, true);
-  return __builtin_bit_cast(double, ((int64_t)hi << 32) | (uint32_t)lo);
-}
-
-__device__ __forceinline__ double lane_read(double x, int lane) {
-  const int64_t b = __builtin_bit_cast(int64_t, x);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xFFFFFFFF), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __builtin_bit_cast(double, ((int64_t)hi << 32) | (uint32_t)lo);
-}
-
-// Maximum over the 64 lanes of a wavefront of values >= 0 (or -1 for none):
-// row shifts inside each row of 16 lanes, then the row broadcasts; lane 63
-// ends with the maximum.
-__device__ __forceinline__ double wave_max_nonneg(double x) {
-  x = fmax(x, dpp_move<0x111, 0xf, 0xf>(x));  // row_shr:1
-  x = fmax(x, dpp_move<0x112, 0xf, 0xf>(x));  // row_shr:2
-  x = fmax(x, dpp_move<0x114, 0xf, 0xe>(x));  // row_shr:4
-  x = fmax(x, dpp_move<0x118, 0xf, 0xc>(x));  // row_shr:8
-  x = fmax(x, dpp_move<0x142, 0xa, 0xf>(x));  // row_bcast:15
-  x = fmax(x, dpp_move<0x143, 0xc, 0xf>(x));  // row_bcast:31
-  return lane_read(x, 63);
-}
-
-// Minimum over the 64 lanes of a wavefront, the same pattern; lanes the masks
-// leave out keep INT_MAX.
-template <int CTRL, int ROWMASK, int BANKMASK>
-__device__ __forceinline__ int dpp_min(int x) {
-  return min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, CTRL, ROWMASK, BANKMASK, false));
-}
-
-__device__ __forceinline__ int wave_min(int x) {
-  x = dpp_min<0x111, 0xf, 0xf>(x);
-  x = dpp_min<0x112, 0xf, 0xf>(x);
-  x = dpp_min<0x114, 0xf, 0xe>(x);
-  x = dpp_min<0x118, 0xf, 0xc>(x);
-  x = dpp_min<0x142, 0xa, 0xf>(x);
-  x = dpp_min<0x143, 0xc, 0xf>(x);
-  return __builtin_amdgcn_readlane(x, 63);
-}
-
 struct FactorShared {
   double l[2][kVankaMaxM];  // the multipliers of the column, by row
   int32_t pr[2], rp[2];     // the pivot's position before the exchange, and its row

@@ -1,5 +1,5 @@
-"""Direct coarse solve on the device (the dense inverse factorised by
-rocSOLVER getrf / getri, applied by k_dense_solve).
+"""Direct coarse solve on the device (the dense inverse, by Gauss-Jordan panels up
+to 1024 unknowns and by rocSOLVER getrf / getri beyond, applied by k_dense_solve).
 
 With ndirect above the finest level's size the whole multigrid is one direct
 solve, so the preconditioner applied to b is A^-1 b: its backward error
@@ -67,3 +67,28 @@ def test_singular_direct_level_is_an_error(ctx):
     h = Hierarchy([lev], 3, "singular")
     with pytest.raises(RuntimeError, match="singular"):
         H.CudaMultiLevelSolver(ctx, h, ndirect=3, **MGP)
+
+
+# around the panels of 32 columns, the 64-row wavefronts and tiles, and the 1024
+# unknowns up to which the inverse is formed by panels
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 65, 100, 257, 1000, 1023, 1024, 1025])
+def test_dense_inverse_sizes(ctx, n):
+    """A one-level direct solve of an orthogonal matrix in random row order with
+    a tiny diagonal (every column needs a row exchange): the residual stays
+    within n 2^-52 |A| |A^-1| |b| (infinity norms), the bound of a solve through
+    an explicit inverse."""
+    print(f"[inverse n={n}]", flush=True)
+    rng = np.random.default_rng(n)
+    A = np.linalg.qr(rng.normal(size=(n, n)))[0]
+    if n > 1:
+        A = A[rng.permutation(n)]
+        np.fill_diagonal(A, 1e-11 * (1 + rng.random(n)))
+    lev = Level(n, 1, np.arange(n + 1, dtype=np.int32) * n,
+                np.tile(np.arange(n, dtype=np.int32), n), A.reshape(-1).copy())
+    mg = H.CudaMultiLevelSolver(ctx, Hierarchy([lev], 3, f"dense{n}"), ndirect=n + 1, **MGP)
+    b = rng.uniform(-1, 1, n)
+    X = mg.new_vector()
+    mg.precondition(X, H.CudaVectorInterface.from_global(ctx, b), x_is_zero=True)
+    r = np.abs(A @ X.copy_back() - b).max()
+    norm = lambda M: np.abs(M).sum(axis=1).max()  # noqa: E731
+    assert r <= n * 2.0 ** -52 * norm(A) * norm(np.linalg.inv(A)) * np.abs(b).max()
