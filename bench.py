@@ -80,11 +80,12 @@ def spmv_bytes(n, nnz, sv, sx):
 
 
 def sell_bytes(n, layout, sv, sx):
-    """bytes of r = b - A x in the device layout: stored values, the column
+    """bytes of r = b - A x in the device layout: stored values (but for the
+    slices that take them from a shared row), the column
     bytes the slices that store columns read (16- or 32-bit; none in pattern
     slices), per-slice metadata (slot, column start, column base: 12 B), one
     16-bit row length or pattern id per row, x once, b, r"""
-    return (layout["stored"] * sv + layout["column_bytes"] + layout["slices"] * 12 + n * 2
+    return ((layout["stored"] - layout["shared"]) * sv + layout["column_bytes"] + layout["slices"] * 12 + n * 2
             + n * sx * 3)
 
 

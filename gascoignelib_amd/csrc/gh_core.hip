@@ -592,6 +592,175 @@ struct KeyTable {
   int64_t fill = 0;
 };
 
+// ------------------------------------------------------------ shared values
+// hash[s]: of the slice's row of values where all its rows follow one pattern
+// and hold the same stored values (never 0), else 0.  One wavefront per slice;
+// a lane without a row repeats the last row's slot.
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void k_sell_hash(int64_t n, int64_t nslices,
+                                                      const uint32_t* __restrict__ sptr,
+                                                      const uint32_t* __restrict__ cptr,
+                                                      const uint32_t* __restrict__ cbase,
+                                                      const int32_t* __restrict__ pstart,
+                                                      const VT* __restrict__ val,
+                                                      uint64_t* __restrict__ hash) {
+  const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
+  if (s >= nslices) return;  // the whole wavefront
+  const int lane = min((int)(threadIdx.x & 63), (int)(n - s * kSlice) - 1);
+  uint64_t h = 0;
+  if ((cptr[s] & 0x60000000u) == 0x60000000u) {
+    const int pid = (int)cbase[s];
+    const int len = pstart[pid + 1] - pstart[pid];
+    h = 0x9E3779B97F4A7C15ull + (uint64_t)pid;
+    for (int k = 0; k < len; ++k) {
+      const double v = (double)ld(val + sptr[s] + (int64_t)k * kSlice + lane);
+      const uint64_t b = __builtin_bit_cast(uint64_t, v);
+      const uint64_t b0 = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) |
+                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(b & 0xFFFFFFFFull));
+      if (__ballot(b != b0)) {
+        h = 0;
+        break;
+      }
+      h = (h ^ b0) * 0xBF58476D1CE4E5B9ull;
+      h ^= h >> 31;
+    }
+    if (__ballot(h != 0)) h |= 1;
+  }
+  if ((threadIdx.x & 63) == 0) hash[s] = h;
+}
+
+// vtab rows from their slices' first rows
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void k_sell_vtab(int64_t nslices,
+                                                      const uint32_t* __restrict__ sptr,
+                                                      const uint32_t* __restrict__ cbase,
+                                                      const int32_t* __restrict__ pstart,
+                                                      const uint32_t* __restrict__ vptr,
+                                                      const int32_t* __restrict__ vrep,
+                                                      const VT* __restrict__ val,
+                                                      SharedT<VT>* __restrict__ vtab) {
+  const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
+  if (s >= nslices || vptr[s] == 0xFFFFFFFFu || vrep[s] != (int32_t)s) return;
+  const int pid = (int)cbase[s];
+  const int len = pstart[pid + 1] - pstart[pid];
+  for (int k = threadIdx.x & 63; k < len; k += kSlice)
+    vtab[vptr[s] + k] = (SharedT<VT>)ld(val + sptr[s] + (int64_t)k * kSlice);
+}
+
+// marks the slices whose rows all hold their vtab row, bit for bit
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void k_sell_mark(int64_t n, int64_t nslices,
+                                                      const uint32_t* __restrict__ sptr,
+                                                      const uint32_t* __restrict__ cbase,
+                                                      const int32_t* __restrict__ pstart,
+                                                      const uint32_t* __restrict__ vptr,
+                                                      const VT* __restrict__ val,
+                                                      const SharedT<VT>* __restrict__ vtab,
+                                                      uint32_t* __restrict__ cptr, int* count) {
+  const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
+  if (s >= nslices || vptr[s] == 0xFFFFFFFFu) return;  // the whole wavefront
+  const int rows = min(kSlice, (int)(n - s * kSlice));
+  const int lane = min((int)(threadIdx.x & 63), rows - 1);
+  const int pid = (int)cbase[s];
+  const int len = pstart[pid + 1] - pstart[pid];
+  bool same = true;
+  for (int k = 0; k < len && same; ++k) {
+    const double a = (double)ld(val + sptr[s] + (int64_t)k * kSlice + lane);
+    const double b = (double)vtab[vptr[s] + k];
+    same = __ballot(__builtin_bit_cast(uint64_t, a) != __builtin_bit_cast(uint64_t, b)) == 0;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    cptr[s] = 0x60000000u | (same ? kSharedBit | vptr[s] : 0u);
+    if (same) atomicAdd(count, rows * len);
+  }
+}
+
+template <typename VT>
+static int sell_share_as(gh_ctx* ctx, const Sell& S, int* count) {
+  const dim3 g(grid_for(S.nslices, kBlock / kSlice)), b(kBlock);
+  hipLaunchKernelGGL(k_sell_vtab<VT>, g, b, 0, ctx->stream, S.nslices, S.sptr, S.cbase, S.pstart,
+                     S.vptr, S.vrep, (const VT*)S.val, (SharedT<VT>*)S.vtab);
+  hipLaunchKernelGGL(k_sell_mark<VT>, g, b, 0, ctx->stream, S.n, S.nslices, S.sptr, S.cbase,
+                     S.pstart, S.vptr, (const VT*)S.val, (const SharedT<VT>*)S.vtab, S.cptr, count);
+  GH_HIP(hipGetLastError());
+  return GH_OK;
+}
+
+int sell_share(gh_ctx* ctx, const Sell& S, int* count) {
+  if (!S.vtab) return GH_OK;
+  if (S.prec == GH_F64) return sell_share_as<double>(ctx, S, count);
+  if (S.prec == GH_F32) return sell_share_as<float>(ctx, S, count);
+  return sell_share_as<__half>(ctx, S, count);
+}
+
+// Finds the slices that share values when the layout is built: slices of one
+// pattern with equal value hashes take one vtab row.
+static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& one) {
+  const int64_t ns = S->nslices;
+  bool any = false;
+  for (int64_t s = 0; s < ns && !any; ++s) any = one[s] != 0;
+  if (!any) return GH_OK;
+  uint64_t* d_hash = nullptr;
+  int* d_count = nullptr;
+  if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * (ns + 1)) != hipSuccess)
+    return fail(GH_ENOMEM, "sell_build: allocation failed");
+  d_count = (int*)(d_hash + ns);
+  std::vector<uint64_t> hash(ns);
+  std::vector<uint32_t> cb(ns), vptr(ns, 0xFFFFFFFFu);
+  std::vector<int32_t> vrep(ns, -1), ps(S->npat + 1);
+  auto run = [&]() -> int {
+    const dim3 g(grid_for(ns, kBlock / kSlice)), b(kBlock);
+    if (S->prec == GH_F64)
+      hipLaunchKernelGGL(k_sell_hash<double>, g, b, 0, ctx->stream, S->n, ns, S->sptr, S->cptr,
+                         S->cbase, S->pstart, (const double*)S->val, d_hash);
+    else if (S->prec == GH_F32)
+      hipLaunchKernelGGL(k_sell_hash<float>, g, b, 0, ctx->stream, S->n, ns, S->sptr, S->cptr,
+                         S->cbase, S->pstart, (const float*)S->val, d_hash);
+    else
+      hipLaunchKernelGGL(k_sell_hash<__half>, g, b, 0, ctx->stream, S->n, ns, S->sptr, S->cptr,
+                         S->cbase, S->pstart, (const __half*)S->val, d_hash);
+    GH_HIP(hipGetLastError());
+    GH_HIP(hipMemsetAsync(d_count, 0, sizeof(int), ctx->stream));
+    GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
+    GH_HIP(hipMemcpyAsync(cb.data(), S->cbase, sizeof(uint32_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
+    GH_HIP(hipMemcpyAsync(ps.data(), S->pstart, sizeof(int32_t) * ps.size(), hipMemcpyDeviceToHost,
+                          ctx->stream));
+    GH_HIP(hipStreamSynchronize(ctx->stream));
+    std::unordered_map<uint64_t, int32_t> first;
+    int64_t total = 0;
+    for (int64_t s = 0; s < ns; ++s) {
+      if (!hash[s]) continue;
+      const int32_t len = ps[cb[s] + 1] - ps[cb[s]];
+      auto it = first.emplace(hash[s], (int32_t)s).first;
+      const int64_t r = it->second;
+      if (r != s && cb[r] != cb[s]) continue;  // equal hashes of two patterns
+      if (r == s) {
+        if (total + len > (int64_t)kSharedMask) continue;
+        vptr[s] = (uint32_t)total;
+        total += len;
+      } else {
+        vptr[s] = vptr[r];
+      }
+      vrep[s] = (int32_t)r;
+    }
+    if (total == 0) return GH_OK;
+    S->nvtab = total;
+    if (hipMalloc(&S->vtab, total * (S->prec == GH_F64 ? 8 : 4)) != hipSuccess)
+      return fail(GH_ENOMEM, "sell_build: allocation failed");
+    GH_TRY(upload(ctx, &S->vptr, vptr.data(), vptr.size()));
+    GH_TRY(upload(ctx, &S->vrep, vrep.data(), vrep.size()));
+    GH_TRY(sell_share(ctx, *S, d_count));
+    int c = 0;
+    GH_HIP(hipMemcpyAsync(&c, d_count, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    GH_HIP(hipStreamSynchronize(ctx->stream));
+    S->shared = (uint32_t)c;
+    return GH_OK;
+  };
+  const int rc = run();
+  (void)hipFree(d_hash);
+  return rc;
+}
+
 static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const uint32_t* col,
                            const double* vals, int prec, const int32_t* orig, Sell* S) {
   S->n = n;
@@ -884,7 +1053,7 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
     (void)hipFree(tmp);
   }
   GH_HIP(hipStreamSynchronize(ctx->stream));
-  return GH_OK;
+  return sell_share_build(ctx, S, one);
 }
 
 // Valued operators: the rows of a window of kSellWindow rows may run in
@@ -1022,8 +1191,11 @@ int sell_build(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const uint32_t* co
 void sell_free(Sell* S) {
   for (void* p : {(void*)S->sptr, (void*)S->rlen, (void*)S->col, S->val, (void*)S->cidx,
                   (void*)S->cptr, (void*)S->cbase, (void*)S->ptab, (void*)S->pstart,
-                  (void*)S->perm})
+                  (void*)S->perm, S->vtab, (void*)S->vptr, (void*)S->vrep})
     if (p) (void)hipFree(p);
+  S->vtab = nullptr;
+  S->vptr = nullptr;
+  S->vrep = nullptr;
   S->perm = nullptr;
   S->ptab = nullptr;
   S->pstart = nullptr;
@@ -1598,10 +1770,17 @@ int csr_asm_commit(gh_ctx* ctx, gh_csr* A, const char* who) {
     hipLaunchKernelGGL(k_sell_refresh<__half>, g, dim3(kBlock), 0, ctx->stream, n, S.sptr, S.perm,
                        A->rowptr, A->d_kept, v64, (__half*)S.val, A->d_flags);
   GH_HIP(hipGetLastError());
+  // which slices share values now; flag [3] counts their entries
+  if (S.vtab) {
+    hipLaunchKernelGGL(k_fill0<int>, dim3(1), dim3(kBlock), 0, ctx->stream, (int64_t)1,
+                       A->d_flags + 3);
+    GH_TRY(sell_share(ctx, S, A->d_flags + 3));
+  }
   int flags[4] = {0, 0, 0, 0};
   GH_HIP(hipMemcpyAsync(flags, A->d_flags, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
   GH_HIP(hipStreamSynchronize(ctx->stream));
   A->h_val_ok = false;
+  A->sell.shared = S.vtab ? (uint32_t)flags[3] : 0;
   if (flags[0] || flags[1] || flags[2]) {
     GH_HIP(hipMemsetAsync(A->d_flags, 0, sizeof(int) * 4, ctx->stream));
     GH_HIP(hipStreamSynchronize(ctx->stream));
@@ -1826,6 +2005,8 @@ int gh_csr_layout(const gh_csr* A, int64_t* out) {
   }
   return GH_OK;
 }
+
+int64_t gh_csr_shared_entries(const gh_csr* A) { return A ? A->sell.shared : 0; }
 
 static int vec_matches(const gh_csr* A, const gh_vec* v) {
   return v && v->n == A->n && v->ncomp == A->ncomp;

@@ -315,6 +315,46 @@ __device__ __forceinline__ T sell_row_pattern(const int32_t* __restrict__ off, u
   return acc;
 }
 
+// One row of a slice whose 64 rows share pattern and values: offsets and values
+// are wave-uniform (scalar loads), the x entry of a step is one load at a scalar
+// base plus the lane's row (n < 2^29 rows, so the byte offset fits 32 bits).  The
+// row length is uniform too, so the last entries' loads are all issued before
+// their steps.  With K > 1, every K-th entry, off and vt at the first of them.
+// No values stream from memory: the residual of the 129^3 constant-coefficient
+// Q1 operator (columns sorted) takes 28 us in FP64 against 87 with its 339 MB of
+// values, 17 in FP32 whatever the storage (f16 21, f32 39); what is left is the
+// vectors, the row order and the x loads from the caches.
+template <int K = 1, typename TV, typename XT, typename T, class Op>
+__device__ __forceinline__ T sell_row_shared(const int32_t* __restrict__ off,
+                                             const TV* __restrict__ vt, uint32_t row, int len,
+                                             const XT* __restrict__ x, T acc, const Op& op) {
+  const uint32_t at = row * (uint32_t)sizeof(XT);
+  auto entry = [&](int k) {
+    return (T) * reinterpret_cast<const XT*>(reinterpret_cast<const char*>(x + off[k * K]) + at);
+  };
+  int k = 0;
+  for (; k + 8 <= len; k += 8) {
+    T xv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) xv[u] = entry(k + u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = op.step(acc, (T)vt[(k + u) * K], xv[u]);
+  }
+  T xv[7];
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (k + u < len) xv[u] = entry(k + u);
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (k + u < len) acc = op.step(acc, (T)vt[(k + u) * K], xv[u]);
+  return acc;
+}
+
+// type of the shared value rows of a storage type
+template <typename VT>
+using SharedT = typename std::conditional<std::is_same<VT, double>::value, double, float>::type;
+constexpr uint32_t kSharedBit = 0x10000000u, kSharedMask = 0x0FFFFFFFu;
+
 // valued operator (matrix); VT storage type, T arithmetic type.  A slice is one
 // wavefront, so the column-encoding branch is uniform across the wave.
 template <typename VT, typename XT, typename T, class Op>
@@ -325,6 +365,7 @@ __global__ __launch_bounds__(kBlock) void k_sell(int64_t n, const uint32_t* __re
                                                  const uint32_t* __restrict__ cbase,
                                                  const int32_t* __restrict__ ptab,
                                                  const int32_t* __restrict__ pstart,
+                                                 const SharedT<VT>* __restrict__ vtab,
                                                  const VT* __restrict__ val,
                                                  const int32_t* __restrict__ perm,
                                                  const XT* __restrict__ x, Op op) {
@@ -346,7 +387,11 @@ __global__ __launch_bounds__(kBlock) void k_sell(int64_t n, const uint32_t* __re
     // one pattern for the whole slice: wave-uniform offsets (scalar loads)
     const int pid = __builtin_amdgcn_readfirstlane((int)cbase[s]);
     const int p0 = pstart[pid];
-    acc = sell_row_pattern(ptab + p0, (uint32_t)row, vp, pstart[pid + 1] - p0, x, acc, op);
+    const int len = pstart[pid + 1] - p0;
+    if (meta & kSharedBit)
+      acc = sell_row_shared(ptab + p0, vtab + (meta & kSharedMask), (uint32_t)row, len, x, acc, op);
+    else
+      acc = sell_row_pattern(ptab + p0, (uint32_t)row, vp, len, x, acc, op);
   } else {
     const int r = rlen[slot];  // entry count, or pattern id in pattern slices
     if (meta & 0x40000000u) {
@@ -377,7 +422,8 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_split(
     int64_t n, const uint32_t* __restrict__ sptr, const uint16_t* __restrict__ rlen,
     const uint16_t* __restrict__ cidx, const uint32_t* __restrict__ cptr,
     const uint32_t* __restrict__ cbase, const int32_t* __restrict__ ptab,
-    const int32_t* __restrict__ pstart, const VT* __restrict__ val,
+    const int32_t* __restrict__ pstart, const SharedT<VT>* __restrict__ vtab,
+    const VT* __restrict__ val,
     const int32_t* __restrict__ perm, const XT* __restrict__ x, Op op) {
   static_assert(!Op::kExact, "split sweeps reorder the row sums");
   __shared__ T part[K][kSlice];
@@ -396,8 +442,12 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_split(
   if ((meta & 0x60000000u) == 0x60000000u) {
     const int pid = __builtin_amdgcn_readfirstlane((int)cbase[s]);
     const int p0 = pstart[pid];
-    acc = sell_row_pattern<K>(ptab + p0 + w, (uint32_t)row, vp, mine(pstart[pid + 1] - p0), x,
-                              acc, op);
+    const int len = mine(pstart[pid + 1] - p0);
+    if (meta & kSharedBit)
+      acc = sell_row_shared<K>(ptab + p0 + w, vtab + (meta & kSharedMask) + w, (uint32_t)row, len,
+                               x, acc, op);
+    else
+      acc = sell_row_pattern<K>(ptab + p0 + w, (uint32_t)row, vp, len, x, acc, op);
   } else {
     const int r = rlen[slot];
     if (meta & 0x40000000u) {
@@ -436,7 +486,8 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_fold(
     int64_t n, const uint32_t* __restrict__ sptr, const uint16_t* __restrict__ rlen,
     const uint16_t* __restrict__ cidx, const uint32_t* __restrict__ cptr,
     const uint32_t* __restrict__ cbase, const int32_t* __restrict__ ptab,
-    const int32_t* __restrict__ pstart, const VT* __restrict__ val,
+    const int32_t* __restrict__ pstart, const SharedT<VT>* __restrict__ vtab,
+    const VT* __restrict__ val,
     const int32_t* __restrict__ perm, const XT* __restrict__ x, Op op) {
   constexpr int E = 8, C = K * E;
   __shared__ T part[2][C][kSlice];
@@ -483,9 +534,17 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_fold(
         c[u] = cb + c16[(int64_t)min(c0 + u * K + w, width - 1) * kSlice];
     }
   };
+  const bool shared = (meta & 0x70000000u) == 0x70000000u;
+  const SharedT<VT>* vt = vtab + (shared ? meta & kSharedMask : 0u);
   auto entries = [&](int c0) {
+    if (shared) {  // (as many entries as the slice is wide, the same for every row)
 #pragma unroll
-    for (int u = 0; u < E; ++u) a[u] = (T)ld(vp + (int64_t)min(c0 + u * K + w, width - 1) * kSlice);
+      for (int u = 0; u < E; ++u) a[u] = (T)vt[min(c0 + u * K + w, width - 1)];
+    } else {
+#pragma unroll
+      for (int u = 0; u < E; ++u)
+        a[u] = (T)ld(vp + (int64_t)min(c0 + u * K + w, width - 1) * kSlice);
+    }
 #pragma unroll
     for (int u = 0; u < E; ++u) xv[u] = (T)x[c[u]];
   };
@@ -644,7 +703,7 @@ template <typename VT, typename XT, typename T, class Op, int K>
 inline int sell_fold_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
   hipLaunchKernelGGL((k_sell_fold<VT, XT, T, Op, K>), dim3((unsigned)S.nslices), dim3(kSlice * K),
                      0, ctx->stream, S.n, S.sptr, S.rlen, S.cidx, S.cptr, S.cbase, S.ptab,
-                     S.pstart, (const VT*)S.val, S.perm, x, op);
+                     S.pstart, (const SharedT<VT>*)S.vtab, (const VT*)S.val, S.perm, x, op);
   GH_HIP(hipGetLastError());
   return GH_OK;
 }
@@ -653,7 +712,7 @@ template <typename VT, typename XT, typename T, class Op, int K>
 inline int sell_split_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
   hipLaunchKernelGGL((k_sell_split<VT, XT, T, Op, K>), dim3((unsigned)S.nslices),
                      dim3(kSlice * K), 0, ctx->stream, S.n, S.sptr, S.rlen, S.cidx, S.cptr,
-                     S.cbase, S.ptab, S.pstart, (const VT*)S.val, S.perm, x, op);
+                     S.cbase, S.ptab, S.pstart, (const SharedT<VT>*)S.vtab, (const VT*)S.val, S.perm, x, op);
   GH_HIP(hipGetLastError());
   return GH_OK;
 }
@@ -678,7 +737,7 @@ inline int sell_launch(gh_ctx* ctx, const Sell& S, const XT* x, Op op) {
   }
   hipLaunchKernelGGL((k_sell<VT, XT, T, Op>), dim3(grid_for(S.n)), dim3(kBlock), 0, ctx->stream,
                      S.n, S.sptr, S.rlen, S.cidx, S.cptr, S.cbase, S.ptab, S.pstart,
-                     (const VT*)S.val, S.perm, x, op);
+                     (const SharedT<VT>*)S.vtab, (const VT*)S.val, S.perm, x, op);
   GH_HIP(hipGetLastError());
   return GH_OK;
 }

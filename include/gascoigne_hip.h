@@ -134,6 +134,9 @@ int gh_csr_prec(const gh_csr* A);
  * 4 out[0], out[7] = 1; other block sizes: out[0] = out[1] = nnz blocks,
  * out[2..5] = 0, out[6] = 4 nnz, out[7] = 0. */
 int gh_csr_layout(const gh_csr* A, int64_t* out);
+/* stored entries whose values a sweep takes from rows shared by whole slices
+ * (a slice whose 64 rows hold equal values stores them, but does not read them) */
+int64_t gh_csr_shared_entries(const gh_csr* A);
 /* The values the device holds, in A's CSR order (nnz*B*B, reduced-precision
  * values widened to FP64); the D2H half of operator<< (print of the device
  * matrix, cuda/cudacsrmatrixinterface.cc:439).  Synchronises. */

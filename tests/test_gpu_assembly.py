@@ -22,7 +22,7 @@ import pytest
 
 from gascoignelib_amd import hip as H
 from gascoignelib_amd import native as N
-from gascoignelib_amd.problem import lattice_rhs
+from gascoignelib_amd.problem import lattice_rhs, lexicographic_order, permuted_csr
 from gascoignelib_amd.structure import Mesh, assemble_hierarchy, coarse_coefficients
 
 pytestmark = pytest.mark.gpu
@@ -221,3 +221,44 @@ def test_solver_reassembly_matches_host_built_solver(ctx, prec, krylov):
         for fp64 in (True, False):
             assert np.array_equal(mg1.level_matrix(l, fp64).values(),
                                   mg2.level_matrix(l, fp64).values())
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+def test_shared_values_follow_the_assembly(ctx, prec):
+    """A matrix created with k = 1 shares its interior rows' values and does so
+    after it was assembled with k = 1 again; one with a layout for varying k is
+    assembled with k = 1, a varying k and k = 1.  Every time the products equal
+    those of a matrix created from the values (to the rounding of the layouts'
+    different sums)."""
+    M = Mesh("cube.inp", 3, 5, 1)
+    l = M.nlevels - 1
+    order = lexicographic_order(M.coords(l))  # rows of one kind side by side
+    inv = np.argsort(order)
+    k = np.random.default_rng(4).uniform(0.5, 2.0, len(M.cells(l)))
+
+    def host(kk):
+        return permuted_csr(assemble_hierarchy(M, kk).fine, order)
+
+    rp, col, val = host(None)
+    n = len(order)
+    cells = H.CoefficientCells(ctx, 3, M.coords(l)[order], inv[M.cells(l)])
+    mask = H.DirichletMask(ctx, n, 1, inv[M.dirichlet(l)])
+    # the pattern of the varying operator: the entries that vanish for k = 1 are
+    # left out of a layout made from it, so the layout is made from their sum
+    A = H.CudaCSRMatrixInterface(ctx, rp, col, val + host(k)[2], prec=prec)
+    B = H.CudaCSRMatrixInterface(ctx, rp, col, val, prec=prec)
+    assert A.layout()["shared"] * 10 < B.layout()["shared"]  # unit rows share in both
+    vp = "f64" if prec == "f64" else "f32"
+    X = H.CudaVectorInterface.from_global(ctx, np.random.default_rng(5).uniform(-1, 1, n), 1, vp)
+    Y, Z = (H.CudaVectorInterface(ctx, n, 1, vp) for _ in range(2))
+    for kk in (None, k, None):
+        K = None if kk is None else H.CudaVectorInterface.from_global(ctx, kk)
+        for C in (A, B) if kk is None else (A,):
+            cells.assemble(C, K, mask)
+            fresh = H.CudaCSRMatrixInterface(ctx, rp, col, host(kk)[2], prec=prec)
+            C.vmult(Y, X)
+            fresh.vmult(Z, X)
+            y, z = Y.copy_back(), Z.copy_back()
+            assert np.abs(y - z).max() <= (1e-14 if prec == "f64" else 1e-5) * np.abs(z).max()
+        if kk is None:
+            assert B.layout()["shared"] > 0

@@ -18,7 +18,9 @@ import scipy.sparse as sp
 import oracle_ctypes as O
 from conftest import fixture_path
 from gascoignelib_amd import hip as H
-from gascoignelib_amd.problem import Hierarchy, splitmix64_uniform
+from gascoignelib_amd.problem import (Hierarchy, lexicographic_order, permuted_csr,
+                                      splitmix64_uniform)
+from gascoignelib_amd.structure import q2_hierarchy, uniform_hierarchy
 
 pytestmark = pytest.mark.gpu
 
@@ -570,6 +572,47 @@ def test_reduced_precision_sweeps_long_rows(ctx, n, L, prec):
         want = x + scale * r
         bound = scale * bound_r + 2.0 ** -21 * (np.abs(x) + np.abs(scale * r))
         assert np.all(np.abs(X.copy_back() - want) <= bound), smoother
+
+
+def sorted_level(kind, refine):
+    """a uniform level in lexicographic order, columns ascending: its interior
+    rows share their relative columns and their values"""
+    if kind == "q1":
+        h = uniform_hierarchy("square.inp" if refine > 6 else "cube.inp", 2 if refine > 6 else 3,
+                              refine)
+    else:
+        h = q2_hierarchy(refine)
+    lev = h.fine
+    return permuted_csr(lev, lexicographic_order(lev.coords)), lev
+
+
+@pytest.mark.parametrize("kind,refine", [("q1", 3), ("q1", 5), ("q1", 7), ("q2", 4), ("q2", 5)])
+def test_shared_values(ctx, kind, refine):
+    """Slices whose 64 rows hold equal values read them from one shared row: the
+    FP64 products keep the oracle's bits, FP32- and FP16-stored ones equal those
+    of a matrix whose slices hardly share (every row scaled by its own power of
+    two, results scaled back), and the layout counts the shared entries."""
+    print(f"[shared {kind} {refine}]", flush=True)
+    (rowptr, col, val), lev = sorted_level(kind, refine)
+    A = H.CudaCSRMatrixInterface(ctx, rowptr, col, val)
+    shared = A.layout()["shared"]
+    assert shared <= np.count_nonzero(val)
+    assert shared > 0 or refine < 5
+    check_products_vs_oracle(ctx, A, rowptr, col, val, refine)
+    n = len(rowptr) - 1
+    scale = 2.0 ** (np.arange(n) % 3)
+    val = val * 1024.0  # no subnormal f16 values
+    sval = val * np.repeat(scale, np.diff(rowptr))
+    x = np.random.default_rng(refine).uniform(-1, 1, n)
+    for prec in ("f32", "f16"):
+        B = H.CudaCSRMatrixInterface(ctx, rowptr, col, val, prec=prec)
+        D = H.CudaCSRMatrixInterface(ctx, rowptr, col, sval, prec=prec)
+        assert B.layout()["shared"] == shared and D.layout()["shared"] * 4 <= shared
+        X = H.CudaVectorInterface.from_global(ctx, x, 1, "f32")
+        Y, Z = (H.CudaVectorInterface(ctx, n, 1, "f32") for _ in range(2))
+        B.vmult(Y, X)
+        D.vmult(Z, X)
+        assert np.array_equal(Y.copy_back(), Z.copy_back() / scale)
 
 
 @pytest.mark.parametrize("n,L", [(90, 33), (700, 40), (5000, 64), (700, 66), (5000, 100), (90, 128),
