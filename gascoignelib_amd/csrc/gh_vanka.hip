@@ -292,86 +292,7 @@ __device__ __forceinline__ T bcast(T v, int lane) {
   }
 }
 
-// one wavefront per patch; rows lane (slot 0) and lane + 64 (slot 1)
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int psize, int B,
-                                                        const int32_t* __restrict__ cls, int ld,
-                                                        const T* __restrict__ lu,
-                                                        const int32_t* __restrict__ gidx,
-                                                        const T* __restrict__ h,
-                                                        T* __restrict__ xp) {
-  const int lane = threadIdx.x & 63;
-  const int64_t p = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  if (p >= npatches) return;  // the whole wavefront
-  const int m = psize * B;
-  const T* L = lu + (int64_t)cls[p] * ld * m;
-  // H = P H: gidx holds, per row of the factors, the global entry that the
-  // recorded row exchanges bring there
-  const int32_t* gi = gidx + p * m;
-  T v0 = (T)0, v1 = (T)0;
-  if (lane < m) v0 = h[gi[lane]];
-  if (lane + 64 < m) v1 = h[gi[lane + 64]];
-  // The column loads of a batch of kBatch steps are issued together, before
-  // the batch's (sequential) updates; every element still sees the same
-  // operations in the same order.  Each pass reads only its triangle: the
-  // forward pass the rows below the diagonal, the backward pass the rows
-  // above it and the diagonal.  (Measured on 32768 patches of 108 unknowns:
-  // batches of 16 beat 8 and 32, and beat double-buffered batches, whose
-  // register cost halves the wavefronts in flight.)
-  constexpr int kBatch = 16;
-  const bool in0 = lane < m, in1 = lane + 64 < m;
-  // unit lower: column k updates rows i > k
-  for (int k0 = 0; k0 < m - 1; k0 += kBatch) {
-    T a0[kBatch], a1[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int k = min(k0 + u, m - 1);
-      const T* Lk = L + (int64_t)k * ld;
-      a0[u] = (in0 && lane > k) ? Lk[lane] : (T)0;
-      a1[u] = (in1 && lane + 64 > k) ? Lk[lane + 64] : (T)0;
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int k = k0 + u;
-      if (k < m - 1) {
-        const T yk = bcast(k < 64 ? v0 : v1, k & 63);
-        if (lane > k && in0) v0 = add_rn(v0, -mul_rn(a0[u], yk));
-        if (lane + 64 > k && in1) v1 = add_rn(v1, -mul_rn(a1[u], yk));
-      }
-    }
-  }
-  // upper: h_k /= u_kk, then column k updates rows i < k
-  for (int k0 = m - 1; k0 >= 0; k0 -= kBatch) {
-    T a0[kBatch], a1[kBatch], dg[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int kk = max(k0 - u, 0);
-      const T* Uk = L + (int64_t)kk * ld;
-      a0[u] = lane < kk ? Uk[lane] : (T)0;
-      a1[u] = lane + 64 < kk ? Uk[lane + 64] : (T)0;
-      dg[u] = Uk[kk];
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int k = k0 - u;
-      if (k >= 0) {
-        if (lane == (k & 63)) {
-          if (k < 64) v0 = v0 / dg[u];
-          else v1 = v1 / dg[u];
-        }
-        const T yk = bcast(k < 64 ? v0 : v1, k & 63);
-        if (lane < k) v0 = add_rn(v0, -mul_rn(a0[u], yk));
-        if (lane + 64 < k) v1 = add_rn(v1, -mul_rn(a1[u], yk));
-      }
-    }
-  }
-  T* out = xp + p * (int64_t)m;
-  if (lane < m) out[lane] = v0;
-  if (lane + 64 < m) out[lane + 64] = v1;
-}
-
-// ------------------------------------------------------------ grouped solve
-// reciprocals of the diagonal of U for the grouped solve's divisions; 0 where
+// reciprocals of the diagonal of U for the solves' divisions; 0 where
 // a plain division is needed (zero or extreme diagonals)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_vanka_rdiag(int64_t nclasses, int m, int ld,
@@ -408,6 +329,151 @@ __device__ __forceinline__ bool in_range(double q) {
 }
 __device__ __forceinline__ bool in_range(float q) { return fabsf(q) <= 3.0e38f; }
 
+// A patch's solve with plain divisions, the local vector in `out`: for patches
+// whose values leave divide_by's range.  The N lanes r = 0 .. N - 1 of one
+// wavefront; its memory operations on one address are ordered once the earlier
+// ones are waited for.
+template <int N, typename T>
+__device__ __attribute__((noinline)) void solve_plain(int m, int ld, const T* L,
+                                                      const int32_t* gi, const T* h,
+                                                      volatile T* out, int r) {
+  for (int i = r; i < m; i += N) out[i] = h[gi[i]];
+  __builtin_amdgcn_s_waitcnt(0);
+  for (int k = 0; k < m - 1; ++k) {
+    const T y = out[k];
+    __builtin_amdgcn_s_waitcnt(0);
+    for (int i = r; i < m; i += N)
+      if (i > k) out[i] = add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+  for (int k = m - 1; k >= 0; --k) {
+    const T y = (T)out[k] / L[k * ld + k];
+    __builtin_amdgcn_s_waitcnt(0);
+    for (int i = r; i <= k; i += N)
+      out[i] = i == k ? y : add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+}
+
+// ------------------------------------------------------------ streamed solve
+// Steps U .. 15 of a batch of 16 columns k0 .. k0 + 15 of the forward pass: column
+// k updates the rows below k.  HI: the columns are 64 and up (rows lane + 64
+// only).  Entries outside the triangle were loaded as zeros and leave their rows
+// as they are, so no step needs a condition.
+template <bool HI, typename T>
+__device__ __forceinline__ void stream_lower(const T (&a0)[16], const T (&a1)[16], int l0, T& v0,
+                                             T& v1) {
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const T y = bcast(HI ? v1 : v0, l0 + u);
+    if (!HI) v0 = add_rn(v0, -mul_rn(a0[u], y));
+    v1 = add_rn(v1, -mul_rn(a1[u], y));
+  }
+}
+
+// One wavefront per patch, rows lane and lane + 64, for patches with factors of
+// their own.  The column loads of a batch of 16 steps are issued together, before
+// the batch's (sequential) updates; each pass reads only its triangle.  Every
+// element sees the oracle's operations in its order (divisions: divide_by).  With
+// many patches the factors' bytes bound it (13824 patches of 108 unknowns: 310 us
+// in FP64, 4.2 TB/s, and 158 in FP32), with few the instructions of the 2 m steps
+// and their loads: masks and branches per load and step, a division per step and
+// the diagonal in vector registers cost as much again (1728 patches in FP32 41
+// instead of 22 us, 13824 in FP64 353).  More batches in flight do not help (4 of
+// 8 columns, 2 or 3 of 16: slower, by their registers).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_vanka_solve(int64_t npatches, int m,
+                                                        const int32_t* __restrict__ cls, int ld,
+                                                        const T* __restrict__ lu,
+                                                        const double* __restrict__ rdiag,
+                                                        const int32_t* __restrict__ gidx,
+                                                        const T* __restrict__ h,
+                                                        T* __restrict__ xp) {
+  const int lane = threadIdx.x & 63;
+  const int64_t p = (int64_t)blockIdx.x * (kBlock / 64) +
+                    __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (p >= npatches) return;  // the whole wavefront
+  const int64_t c = cls[p];
+  const T* L = lu + c * ld * m;
+  const double* rd = rdiag + c * m;
+  // H = P H: gidx holds, per row of the factors, the global entry that the
+  // recorded row exchanges bring there
+  const int32_t* gi = gidx + p * m;
+  const bool in0 = lane < m, in1 = lane + 64 < m;
+  T v0 = in0 ? h[gi[lane]] : (T)0;
+  T v1 = in1 ? h[gi[lane + 64]] : (T)0;
+  const int last = m - 1;
+  // Rows and columns past the matrix are zeros (columns past it repeat the last,
+  // with y = 0), so only the 16 x 16 blocks on the diagonal need a mask per step;
+  // lanes outside a batch's rows leave the loads as a whole.
+  // unit lower: column k updates rows i > k
+  for (int k0 = 0; k0 < last; k0 += 16) {
+    const bool hi = k0 >= 64;
+    T a0[16] = {}, a1[16] = {};
+    if (!hi && lane >= k0 && lane < ld) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a0[u] = L[(int64_t)min(k0 + u, last) * ld + lane];
+    }
+    if (lane + 64 >= k0 && lane + 64 < ld) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a1[u] = L[(int64_t)min(k0 + u, last) * ld + lane + 64];
+    }
+    if (!hi) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a0[u] = lane > k0 + u ? a0[u] : (T)0;
+      stream_lower<false>(a0, a1, k0, v0, v1);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a1[u] = lane + 64 > k0 + u ? a1[u] : (T)0;
+      stream_lower<true>(a0, a1, k0 - 64, v0, v1);
+    }
+  }
+  // upper: h_k /= u_kk, then column k updates rows i < k
+  for (int k0 = last & ~15; k0 >= 0; k0 -= 16) {
+    const bool hi = k0 >= 64;
+    T a0[16] = {}, a1[16] = {};
+    // lane u keeps column k0 + u's diagonal and its reciprocal
+    const int kd = min(k0 + (lane & 15), last);
+    const double dl = (double)L[(int64_t)kd * (ld + 1)], rl = rd[kd];
+    if (lane < k0 + 16 && lane < ld) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a0[u] = L[(int64_t)min(k0 + u, last) * ld + lane];
+    }
+    if (hi && lane + 64 < k0 + 16) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a1[u] = L[(int64_t)min(k0 + u, last) * ld + lane + 64];
+    }
+    if (hi) {
+#pragma unroll
+      for (int u = 15; u >= 0; --u) {
+        const T q = divide_by(v1, lane_read(dl, u), lane_read(rl, u));
+        const T y = bcast(q, k0 - 64 + u);
+        const T a = lane + 64 < k0 + u ? a1[u] : (T)0;
+        v1 = lane + 64 == k0 + u ? q : add_rn(v1, -mul_rn(a, y));
+        v0 = add_rn(v0, -mul_rn(a0[u], y));
+      }
+    } else {
+#pragma unroll
+      for (int u = 15; u >= 0; --u) {
+        const T q = divide_by(v0, lane_read(dl, u), lane_read(rl, u));
+        const T y = bcast(q, k0 + u);
+        const T a = lane < k0 + u ? a0[u] : (T)0;
+        v0 = lane == k0 + u ? q : add_rn(v0, -mul_rn(a, y));
+      }
+    }
+  }
+  T* out = xp + p * (int64_t)m;
+  const bool ok = (!in0 || (in_range(v0) && rd[lane] != 0.0)) &&
+                  (!in1 || (in_range(v1) && rd[lane + 64] != 0.0));
+  if (__builtin_expect(__ballot(!ok) != 0, 0)) {
+    solve_plain<64>(m, ld, L, gi, h, out, lane);
+    return;
+  }
+  if (in0) out[lane] = v0;
+  if (in1) out[lane + 64] = v1;
+}
+
+// ------------------------------------------------------------- grouped solve
 // lane N of each 16-lane row, to the whole row
 template <int N>
 __device__ __forceinline__ float row_bcast(float x) {
@@ -523,32 +589,6 @@ __device__ __forceinline__ void group_backward(const T* __restrict__ L,
 // zeros up to column 16 MB
 __host__ __device__ constexpr int group_entries(int mb) { return 256 * mb * mb; }
 
-// The same solve with plain divisions, the local vector in `out`: for patches
-// whose values leave divide_by's range.  16 lanes of one wavefront; a wavefront's
-// memory operations on one address are ordered once the earlier ones are waited
-// for.
-template <typename T>
-__device__ __attribute__((noinline)) void solve_plain(int m, int ld, const T* L,
-                                                      const int32_t* gi, const T* h,
-                                                      volatile T* out, int r) {
-  for (int i = r; i < m; i += 16) out[i] = h[gi[i]];
-  __builtin_amdgcn_s_waitcnt(0);
-  for (int k = 0; k < m - 1; ++k) {
-    const T y = out[k];
-    __builtin_amdgcn_s_waitcnt(0);
-    for (int i = r; i < m; i += 16)
-      if (i > k) out[i] = add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
-    __builtin_amdgcn_s_waitcnt(0);
-  }
-  for (int k = m - 1; k >= 0; --k) {
-    const T y = (T)out[k] / L[k * ld + k];
-    __builtin_amdgcn_s_waitcnt(0);
-    for (int i = r; i <= k; i += 16)
-      out[i] = i == k ? y : add_rn((T)out[i], -mul_rn(L[k * ld + i], y));
-    __builtin_amdgcn_s_waitcnt(0);
-  }
-}
-
 // Patches of one class per workgroup: the factors go to LDS once (16-byte
 // loads, the first local vectors gathered meanwhile), then 16 lanes solve each
 // patch, lane r holding its rows r, r + 16, ... (MB of them), the solved value
@@ -630,7 +670,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_vanka_group(int m, int64_t ls
     for (int j = 0; j < MB; ++j) ok = ok && in_range(v[j]);
     const uint64_t bad = __ballot(!ok) >> (threadIdx.x & 48);
     if (__builtin_expect((bad & 0xFFFF) != 0, 0)) {
-      solve_plain<T>(m, 16 * MB, lu + c * lstride, gidx + p * m, h, out, r);
+      solve_plain<16>(m, 16 * MB, lu + c * lstride, gidx + p * m, h, out, r);
     } else {
 #pragma unroll
       for (int j = 0; j < MB; ++j)
@@ -712,7 +752,7 @@ int vanka_apply_t(gh_ctx* ctx, const gh_vanka* V, const T* in, T* out, int mode,
   } else {
     const unsigned gs = (unsigned)((V->npatches + kBlock / 64 - 1) / (kBlock / 64));
     hipLaunchKernelGGL(k_vanka_solve<T>, dim3(gs), dim3(kBlock), 0, ctx->stream, V->npatches,
-                       V->psize, V->B, V->cls, V->ld, (const T*)V->lu, V->piv, in, (T*)V->xp);
+                       V->m, V->cls, V->ld, (const T*)V->lu, V->rdiag, V->piv, in, (T*)V->xp);
   }
   const unsigned ga = (unsigned)((V->n * V->B + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(k_vanka_average<T>, dim3(ga), dim3(kBlock), 0, ctx->stream, V->n, V->B,
@@ -807,7 +847,7 @@ int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
   const int64_t at_once = fit * ctx->num_cu;
   // Distinct factors are read once either way: the grouped solve is faster while
   // every patch has a workgroup at once (216 patches of 108 unknowns 16 us
-  // against 36 in FP32, 1728 patches 69 against 42), shared factors always.
+  // against 36 in FP32, 1728 patches 69 against 22), shared factors always.
   if (np < 2 * nc && np > at_once) return GH_OK;
   if (!(V->prec == GH_F64 ? group_allow<double>(V->m) : group_allow<float>(V->m))) {
     (void)hipGetLastError();
