@@ -382,6 +382,11 @@ int hn_apply(gh_ctx* ctx, const gh_hn* H, int ncomp, int prec, void* x, int op);
 int mask_apply(gh_ctx* ctx, const gh_mask* M, int prec, void* x);
 int mgs_step(gh_ctx* ctx, int64_t size, double* vv, const double* prev, int dslot,
              const double* next, int oslot);
+// the whole step in one launch for vectors that mgs_is_small: scal[slot0 + k] =
+// <vv, basis[k]> (k < dim, vv updated in between), scal[slot0 + dim] = <vv, vv>
+bool mgs_is_small(int64_t size);
+int mgs_small(gh_ctx* ctx, int64_t size, double* vv, const double* const* dbasis, int dim,
+              int slot0);
 int finalize_slots(gh_ctx* ctx, int first, int count, bool max);
 // classical Gram-Schmidt: scal[slot0 + k] = <w, basis[k]> (k < dim); then
 // w -= sum_k scal[hslot0 + k] basis[k] and scal[oslot] = <w, w>

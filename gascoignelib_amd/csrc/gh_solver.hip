@@ -1223,10 +1223,15 @@ int arnoldi_step(gh_mg* mg, int dim, double* vv, std::vector<double>& h,
     h[dim] = std::sqrt(d[dim]);
   }
   for (int pass = 0; pass < 2 && !classical; ++pass) {
-    GH_TRY(mgs_step(ctx, n, vv, nullptr, 0, mg->mem[0], 8));
-    for (int i = 1; i < dim; ++i) GH_TRY(mgs_step(ctx, n, vv, mg->mem[i - 1], 8 + i - 1, mg->mem[i], 8 + i));
-    GH_TRY(mgs_step(ctx, n, vv, mg->mem[dim - 1], 8 + dim - 1, nullptr, 8 + dim));
-    GH_TRY(finalize_slots(ctx, 8, dim + 1, false));
+    if (mgs_is_small(n)) {
+      GH_TRY(mgs_small(ctx, n, vv, (const double* const*)mg->d_basis, dim, 8));
+    } else {
+      GH_TRY(mgs_step(ctx, n, vv, nullptr, 0, mg->mem[0], 8));
+      for (int i = 1; i < dim; ++i)
+        GH_TRY(mgs_step(ctx, n, vv, mg->mem[i - 1], 8 + i - 1, mg->mem[i], 8 + i));
+      GH_TRY(mgs_step(ctx, n, vv, mg->mem[dim - 1], 8 + dim - 1, nullptr, 8 + dim));
+      GH_TRY(finalize_slots(ctx, 8, dim + 1, false));
+    }
     GH_TRY(fetch_scalars(ctx, 8, dim + 1, d.data()));
     for (int i = 0; i < dim; ++i) h[i] += d[i];
     h[dim] = std::sqrt(d[dim]);

@@ -299,6 +299,55 @@ def test_gmres_vs_oracle(ctx, name):
     assert ig.residual == pytest.approx(io.residual, rel=1e-9)
 
 
+def grid_inp(path, nx, ny):
+    """UCD mesh of nx x ny unit quadrilaterals with boundary colour 1."""
+    node = lambda i, j: j * (nx + 1) + i
+    lines = []
+    for j in range(ny):
+        for i in range(nx):
+            lines.append("0 quad %d %d %d %d" % (node(i, j), node(i + 1, j), node(i + 1, j + 1),
+                                                 node(i, j + 1)))
+    edges = [(node(i, j), node(i + 1, j)) for j in (0, ny) for i in range(nx)]
+    edges += [(node(i, j), node(i, j + 1)) for i in (0, nx) for j in range(ny)]
+    lines += ["1 line %d %d" % e for e in edges]
+    with open(path, "w") as f:
+        f.write("%d %d 0 0 0\n" % ((nx + 1) * (ny + 1), len(lines)))
+        for j in range(ny + 1):
+            for i in range(nx + 1):
+                f.write("%d %d %d 0\n" % (node(i, j), i, j))
+        for k, line in enumerate(lines):
+            f.write("%d %s\n" % (k, line))
+    return str(path)
+
+
+@pytest.mark.parametrize("nx,ny", [(3, 3), (15, 16), (12, 20), (31, 32), (8, 120), (40, 50),
+                                   (27, 74), (49, 41)])
+def test_gmres_vector_lengths(ctx, tmp_path, nx, ny):
+    """GMRES against the oracle where the Gram-Schmidt step changes its form:
+    49 unknowns, 1023 and 1025 around one entry per thread of the single
+    workgroup, 4095 and 4097 around four, 8181 within and 8195 and 8217 beyond
+    eight, where every basis vector is a launch.  Only the order of the sums
+    differs, as in test_gmres_vs_oracle, whose bounds these are."""
+    print(f"[{nx}x{ny}]", flush=True)
+    h = uniform_hierarchy(grid_inp(tmp_path / "grid.inp", nx, ny), 2, 1, 0)
+    assert h.levels[-1].n == (2 * nx + 1) * (2 * ny + 1)
+    mg = H.CudaMultiLevelSolver(ctx, h, ndirect=1, **MGP)
+    om = O.MG(h, ndirect=1, **MGP)
+    f = rhs(h)
+    for steps in (1, 8):
+        io = O.cginfo(1e-30, 1e-300, steps)
+        xo = np.zeros_like(f)
+        om.gmres(xo, f, io, vmax=10)
+        ig = H.CGInfo(1e-30, 1e-300, steps)
+        X = mg.new_vector()
+        mg.Gmres(X, vec(ctx, f), ig, vmax=10)
+        assert ig.iteration == io.iteration
+        assert relerr(X.copy_back(), xo) <= 1e-12
+        # 8 steps leave the 25 free unknowns of 3x3 a residual of rounding size
+        assert ig.residual == pytest.approx(io.residual, rel=1e-9,
+                                            abs=1e-13 * np.linalg.norm(f))
+
+
 @pytest.mark.parametrize("name", FIXTURES)
 def test_newton_solve_vs_oracle(ctx, name):
     """StdMultiLevelSolver::Solve (Newton + GMRES(10) + V(2,2) Jacobi) to 1e-10."""
