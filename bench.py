@@ -85,7 +85,8 @@ def sell_bytes(n, layout, sv, sx):
     bytes the slices that store columns read (16- or 32-bit; none in pattern
     slices), per-slice metadata (slot, column start, column base: 12 B), one
     16-bit row length or pattern id per row, x once, b, r"""
-    return ((layout["stored"] - layout["shared"]) * sv + layout["column_bytes"] + layout["slices"] * 12 + n * 2
+    own = layout["stored"] - layout.get("shared", 0)
+    return (own * sv + layout["column_bytes"] + layout["slices"] * 12 + n * 2
             + n * sx * 3)
 
 
