@@ -10,7 +10,9 @@
 // MgInterpolatorMatrix::restrict_zero / prolongate_add,
 // src/Discretization/Q1/mginterpolatormatrix.cc:123-147).  Reduced-precision
 // (non-exact) sweeps over levels of few slices may instead split a slice over
-// K wavefronts (k_sell_split).
+// K wavefronts (k_sell_split); exact sweeps of long rows form the products in
+// several wavefronts and fold them in the stored order (k_sell_fold).  A slice
+// whose rows share pattern and values reads one row of values (kSharedBit).
 #pragma once
 
 #include <type_traits>
