@@ -1,7 +1,7 @@
 // Direct solve of the coarsest multigrid levels: the dense inverse of the
 // level matrix, formed on the device (Gauss-Jordan with partial pivoting in
-// panels of 32 columns up to 1024 unknowns; beyond, LU with partial pivoting and
-// the inverse from it, rocSOLVER getrf / getri) and applied by k_dense_solve.
+// panels of 32 columns for scalar levels of up to 1024 unknowns; else LU with
+// partial pivoting and the inverse from it, rocSOLVER getrf / getri) and applied by k_dense_solve.
 // The reference solves its coarse level with UMFPACK when it is built with it
 // (src/LinAlg/umfilu.cc, StdSolver::DirectSolver) and otherwise with
 // iterexact smoothing sweeps; any exact solve gives the same V-cycle up to
@@ -309,7 +309,12 @@ int dense_inverse_device(gh_ctx* ctx, const gh_csr* A, double* inv) {
   if (m == 0) return GH_OK;
   if (m > 46340) return fail(GH_EINVAL, "direct coarse level: %lld unknowns is too many for a "
                                         "dense inverse", (long long)m);
-  if (m <= kGjMax) return gj_inverse(ctx, A, m, inv);
+  // Scalar levels only.  The coarsest Stokes-LPS levels of a channel (27 to 81 nodes,
+  // one layer of patches) are singular to rounding (condition 2e16 to 1e17): what
+  // their inverse holds is rounding of the elimination, so they keep the one whose
+  // results their solvers have had so far.  Nothing is lost on the solve: both
+  // inverses are applied by the same kernel.
+  if (B == 1 && m <= kGjMax) return gj_inverse(ctx, A, m, inv);
   if (!ctx->blas) {
     rocblas_handle h = nullptr;
     if (rocblas_create_handle(&h) != rocblas_status_success)
