@@ -721,17 +721,22 @@ int group_launch(gh_ctx* ctx, const gh_vanka* V, const T* h) {
   return GH_OK;
 }
 
-// the LDS of the grouped solve for local systems of m unknowns, allowed once
-// at creation
+// Workgroups of the grouped solve for local systems of m unknowns that a CU holds
+// at once (LDS, registers and wavefronts; 0: none); their LDS is allowed here.
 template <typename T>
-bool group_allow(int m) {
+int group_fit(int m) {
   const int mb = (m + 15) / 16;
   const void* k[8] = {(const void*)k_vanka_group<T, 1>, (const void*)k_vanka_group<T, 2>,
                       (const void*)k_vanka_group<T, 3>, (const void*)k_vanka_group<T, 4>,
                       (const void*)k_vanka_group<T, 5>, (const void*)k_vanka_group<T, 6>,
                       (const void*)k_vanka_group<T, 7>, (const void*)k_vanka_group<T, 8>};
-  return hipFuncSetAttribute(k[mb - 1], hipFuncAttributeMaxDynamicSharedMemorySize,
-                             group_entries(mb) * (int)sizeof(T)) == hipSuccess;
+  const int lds = group_entries(mb) * (int)sizeof(T);
+  int fit = 0;
+  if (hipFuncSetAttribute(k[mb - 1], hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess &&
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k[mb - 1], kGroupThreads, lds) == hipSuccess)
+    return fit;
+  (void)hipGetLastError();
+  return 0;
 }
 
 template <typename T>
@@ -837,27 +842,50 @@ int patch_classes(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, int
   return GH_OK;
 }
 
-// Whether the grouped solve runs, and its groups.
+// Whether the grouped solve runs, and its groups: chunks of a class's patches, as
+// many per workgroup as make the solve shortest.  A workgroup stages its factors
+// (taken as long as one pass) and then solves 32 patches per pass; workgroups
+// beyond those the chip holds at once wait for a place.  (32768 patches of 108
+// unknowns in 27 classes, FP64, one workgroup per CU: 128 patches each would be 270
+// workgroups and a second round for the last 14.)
+//
+// Against the streamed solve the groups must hold enough patches for the factors
+// staged: with one patch each they are slower for any number of patches (108
+// unknowns, 64 patches 24.3 against 23.6 us in FP64; 512 in FP32 27.4 against
+// 22.0), with two where a wavefront of the streamed solve has no second row per
+// lane (m <= 64: 2048 patches of 36, FP64, 13.4 against 16.9; 81 unknowns, FP32,
+// 25.6 against 22.3), with three beyond (108, 512 patches, 21.3 against 27.5).  Once
+// the workgroups come in rounds, a CU that holds few of them waits for their
+// staging, so there it is patches per place of a CU: 108 unknowns in FP64 (one
+// workgroup per CU), 2048 patches in classes of 2, 3, 4, 5 and 8: 83, 59, 43, 42 and
+// 25 us against 40, 44, 38, 44 and 38; 81 unknowns (two per CU), 8192 patches in
+// classes of 2, 3, 4: 139, 103, 76 against 106, 102, 100; 54 unknowns, classes of 2:
+// 54 against 59.
 int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
   const int64_t np = V->npatches, nc = V->nclasses;
-  const int mb = (V->m + 15) / 16;
-  const int64_t ts = V->prec == GH_F64 ? 8 : 4;
-  const int64_t lds = group_entries(mb) * ts + 256 * mb;
-  const int64_t fit = std::min<int64_t>(8, (160 << 10) / lds);  // workgroups a CU holds
+  const int64_t fit = V->prec == GH_F64 ? group_fit<double>(V->m) : group_fit<float>(V->m);
+  if (fit < 1) return GH_OK;
   const int64_t at_once = fit * ctx->num_cu;
-  // Distinct factors are read once either way: the grouped solve is faster while
-  // every patch has a workgroup at once (216 patches of 108 unknowns 16 us
-  // against 36 in FP32, 1728 patches 69 against 22), shared factors always.
-  if (np < 2 * nc && np > at_once) return GH_OK;
-  if (!(V->prec == GH_F64 ? group_allow<double>(V->m) : group_allow<float>(V->m))) {
-    (void)hipGetLastError();
-    return GH_OK;
-  }
-  // a wavefront takes 4 patches at a time: as many per workgroup as fill the
-  // chip once, over 8 wavefronts
-  const int64_t chunk = 4 * std::max<int64_t>(1, (np + 4 * at_once - 1) / (4 * at_once));
   std::vector<int64_t> start(nc + 1, 0);
   for (int64_t p = 0; p < np; ++p) start[cls[p] + 1]++;
+  const int64_t most = *std::max_element(start.begin(), start.end());
+  constexpr int64_t kPass = kGroupThreads / 16;  // patches per pass
+  const int64_t least = V->m > 64 ? 3 : 2;       // patches per group
+  int64_t chunk = 0, ng = 0, best = 0;
+  for (int64_t c = 4;; c += c < kPass ? 4 : kPass) {  // a wavefront takes 4 patches
+    int64_t g = 0;
+    for (int64_t k = 1; k <= nc; ++k) g += (start[k] + c - 1) / c;
+    const int64_t cost = ((g + at_once - 1) / at_once) * (1 + (c + kPass - 1) / kPass);
+    if (chunk == 0 || cost < best || (cost == best && np < least * ng)) {
+      chunk = c;
+      ng = g;
+      best = cost;
+    }
+    // no larger chunk is shorter: one group per class is the least there can be
+    const int64_t rounds = (nc + at_once - 1) / at_once;
+    if (c >= most || (g <= at_once && np >= least * g) || rounds * (2 + c / kPass) > best) break;
+  }
+  if (np < least * ng || (ng > at_once && np * fit < (least + 2) * ng)) return GH_OK;
   for (int64_t c = 0; c < nc; ++c) start[c + 1] += start[c];
   std::vector<int32_t> plist(np), groups;
   {
@@ -1044,6 +1072,8 @@ int gh_vanka_destroy(gh_vanka* V) {
   if (ctx) ctx_release(ctx);
   return GH_OK;
 }
+
+int64_t gh_vanka_groups(const gh_vanka* V) { return V ? V->ngroups : 0; }
 
 int gh_vanka_solve(gh_ctx* ctx, const gh_vanka* V, gh_vec* x) {
   GH_ARG(ctx && V && x, "gh_vanka_solve: NULL argument");

@@ -688,6 +688,11 @@ class VankaSmoother:
     def solve(self, x):
         check(N.hip().gh_vanka_solve(self.ctx.h, self.h, x.h))
 
+    def groups(self):
+        """workgroups of the solve that share factors between equal patches, 0
+        where every patch reads its own"""
+        return int(N.hip().gh_vanka_groups(self.h))
+
     def __del__(self):
         try:
             if self.h:

@@ -140,6 +140,7 @@ HIP_SIGNATURES = {
                                   P(GhNLInfo), C.c_int, P(GhSolveReport)]),
     "gh_vanka_create": (C.c_int, [vp, vp, C.c_int64, C.c_int, i32p, C.c_int, P(vp)]),
     "gh_vanka_destroy": (C.c_int, [vp]),
+    "gh_vanka_groups": (C.c_int64, [vp]),
     "gh_vanka_solve": (C.c_int, [vp, vp, vp]),
     "gh_mg_set_vanka": (C.c_int, [vp, C.c_int, C.c_int64, C.c_int, i32p]),
     "gh_ilu_create": (C.c_int, [vp, vp, i32p, P(vp)]),

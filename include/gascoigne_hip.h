@@ -179,6 +179,9 @@ int gh_jacobi_noalloc(gh_ctx* ctx, const gh_csr* A, gh_vec* h);
 int gh_vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize,
                     const int32_t* nodes, int prec, gh_vanka** out);
 int gh_vanka_destroy(gh_vanka* V);
+/* workgroups of the solve that share factors between patches with equal
+ * matrices; 0: every patch reads its own (the results are the same) */
+int64_t gh_vanka_groups(const gh_vanka* V);
 /* solve (:193-237), in place: x <- (1/count_i) sum_p R_p^T A_p^-1 R_p x, the
  * patches of a node summed in ascending order.  x in the factors' precision. */
 int gh_vanka_solve(gh_ctx* ctx, const gh_vanka* V, gh_vec* x);

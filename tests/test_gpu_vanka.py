@@ -123,8 +123,8 @@ def plane_problem(refine, B, seed, vary, children=4):
 
 
 # local systems of 9 .. 125 unknowns (1 to 8 rows per lane, full and partial),
-# patches that share factors and patches that do not, and more distinct patches
-# than the grouped solve takes (16,384: one wavefront per patch)
+# patches that share factors and patches that do not (one wavefront each), up to
+# 16,384 of them
 @pytest.mark.parametrize("prec", ["f64", "f32"])
 @pytest.mark.parametrize("B,refine,vary,children",
                          [(1, 2, True, 4), (1, 4, False, 4), (2, 4, True, 4), (4, 3, False, 4),
@@ -145,7 +145,7 @@ def test_vanka_solve_shapes(ctx, prec, B, refine, vary, children):
         assert np.abs(X.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
 
 
-# factors and vectors outside the range in which the grouped solve multiplies by
+# factors and vectors outside the range in which the solves multiply by
 # reciprocals: those patches are solved with plain divisions
 @pytest.mark.parametrize("ascale,xscale", [(2.0 ** 500, 1.0), (2.0 ** -450, 2.0 ** -300),
                                            (1.0, 2.0 ** -800), (1.0, 2.0 ** 700)])
@@ -159,3 +159,92 @@ def test_vanka_solve_extreme_values(ctx, ascale, xscale):
     xo = x.copy()
     O.Vanka(O.Matrix(lev.rowptr, lev.col, val, 2), pat).solve(xo)
     assert np.array_equal(X.copy_back(), xo)
+
+
+def class_problem(psize, B, npatches, nclasses, seed, band=None):
+    """disjoint patches of `psize` nodes with `nclasses` different matrices in
+    turn (full, or `band` nodes on each side of the diagonal), whose LU exchanges
+    rows"""
+    r = np.random.default_rng(seed)
+    blk = r.uniform(-1, 1, (nclasses, psize, psize, B, B))
+    i = np.arange(psize)
+    keep = np.abs(i[:, None] - i[None]) <= (psize if band is None else band)
+    rows, cols = np.nonzero(keep)
+    n = npatches * psize
+    rowptr = np.concatenate([[0], np.cumsum(np.tile(keep.sum(1), npatches))]).astype(np.int32)
+    col = (np.arange(npatches)[:, None] * psize + cols[None]).reshape(-1).astype(np.int32)
+    val = blk[np.arange(npatches) % nclasses][:, rows, cols].reshape(-1)
+    return rowptr, col, val, np.arange(n, dtype=np.int32).reshape(npatches, psize), r
+
+
+def check_vanka(ctx, rowptr, col, val, B, patches, x, prec, grouped):
+    """the solve against the oracle: bit for bit in FP64; FP32 factors within what
+    their rounding gives each patch, n_p 2^-24 times the condition of its matrix
+    (times 4: factors, both triangles and the right-hand side)"""
+    V = H.VankaSmoother(ctx, H.CudaCSRMatrixInterface(ctx, rowptr, col, val, B), patches, prec)
+    assert (V.groups() > 0) == grouped
+    X = H.CudaVectorInterface.from_global(ctx, x, B, prec)
+    V.solve(X)
+    xo = x.copy()
+    O.Vanka(O.Matrix(rowptr, col, val, B), patches).solve(xo)
+    if prec == "f64":
+        assert np.array_equal(X.copy_back(), xo)
+        return V
+    P, m = len(patches), patches.shape[1] * B
+    got, want = X.copy_back().reshape(P, m), xo.reshape(P, m)
+    nc = min(P, 8)  # the classes come in turn
+    A = np.zeros((nc, m, m))
+    for p in range(nc):
+        for a in range(patches.shape[1]):
+            for q in range(rowptr[patches[p, a]], rowptr[patches[p, a] + 1]):
+                b = col[q] - patches[p, 0]
+                A[p, a * B:(a + 1) * B, b * B:(b + 1) * B] = val[q * B * B:(q + 1) * B * B].reshape(B, B)
+    cond = np.array([np.linalg.cond(a) for a in A])
+    for p in range(nc):
+        bound = 4 * m * 2.0 ** -24 * cond[p] * np.linalg.norm(want[p])
+        assert np.linalg.norm(got[p] - want[p]) <= bound
+    return V
+
+
+# local systems around the 16-row and 16-column batches and the second row of a
+# lane (64, 65), each with a matrix of its own per patch (streamed) and with 8
+# patches to a matrix (grouped)
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("psize,B", [(1, 1), (2, 1), (15, 1), (16, 1), (17, 1), (31, 1), (16, 2),
+                                     (11, 3), (16, 3), (7, 7), (9, 7), (16, 4), (13, 5), (16, 5),
+                                     (27, 3), (24, 4), (97, 1), (27, 4), (28, 4), (113, 1),
+                                     (25, 5), (127, 1), (32, 4)])
+def test_vanka_solve_both_kernels(ctx, prec, psize, B):
+    print(f"[vanka both {psize}x{B} {prec}]", flush=True)
+    for npatches, nclasses in ((41, 41), (40, 5)):
+        rowptr, col, val, pat, r = class_problem(psize, B, npatches, nclasses, 10 * psize + B)
+        x = r.uniform(-1, 1, npatches * psize * B)
+        check_vanka(ctx, rowptr, col, val, B, pat, x, prec, nclasses < npatches)
+
+
+# more workgroups than the chip holds at once: few patches to a matrix are
+# streamed, enough are grouped; and more than 32 patches to a workgroup
+@pytest.mark.parametrize("psize,B,npatches,nclasses,prec,grouped",
+                         [(9, 1, 4096, 4096, "f64", False), (9, 1, 4096, 2048, "f64", True),
+                          (27, 4, 1600, 800, "f64", False), (27, 4, 1600, 200, "f64", True),
+                          (27, 4, 3200, 1600, "f32", False), (27, 4, 3200, 320, "f32", True),
+                          (27, 4, 8200, 1, "f64", True)])
+def test_vanka_solve_many_patches(ctx, psize, B, npatches, nclasses, prec, grouped):
+    print(f"[vanka {npatches} patches, {nclasses} matrices, {psize}x{B} {prec}]", flush=True)
+    rowptr, col, val, pat, r = class_problem(psize, B, npatches, nclasses, 3, band=1)
+    x = r.uniform(-1, 1, npatches * psize * B)
+    V = check_vanka(ctx, rowptr, col, val, B, pat, x, prec, grouped)
+    if nclasses == 1:
+        assert 32 * V.groups() < npatches
+
+
+# the plain divisions of both kernels, with one and two rows per lane
+@pytest.mark.parametrize("ascale,xscale", [(2.0 ** 500, 1.0), (2.0 ** -450, 2.0 ** -300),
+                                           (1.0, 2.0 ** -800), (1.0, 2.0 ** 700)])
+@pytest.mark.parametrize("psize,B", [(9, 2), (27, 4)])
+def test_vanka_extreme_values_both_kernels(ctx, psize, B, ascale, xscale):
+    for npatches, nclasses in ((17, 17), (24, 3)):
+        rowptr, col, val, pat, r = class_problem(psize, B, npatches, nclasses, 8)
+        x = r.uniform(-1, 1, npatches * psize * B) * xscale
+        x[::3] = 0.0
+        check_vanka(ctx, rowptr, col, val * ascale, B, pat, x, "f64", nclasses < npatches)
