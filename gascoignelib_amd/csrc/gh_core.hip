@@ -382,9 +382,14 @@ int vec_fill_zero(gh_ctx* ctx, int prec, int64_t size, void* x) {
 // block matrices (ncomp > 1): one thread per block row component
 template <int B, typename VT, typename XT, typename Acc, class Op>
 static void launch_bsell_as(gh_ctx* ctx, const BSell& S, const XT* x, Op op) {
-  hipLaunchKernelGGL((k_bsell<B, VT, XT, Acc, Op>), dim3((unsigned)S.nslices),
-                     dim3(64 * kBSplit), 0, ctx->stream, S.sptr, S.row, S.rlen, S.col,
-                     (const VT*)S.val, x, op);
+  if (bsell_is_split(S))
+    hipLaunchKernelGGL((k_bsell_split<B, VT, XT, Acc, Op>), dim3((unsigned)S.nslices),
+                       dim3(64 * kBSplit), 0, ctx->stream, S.sptr, S.row, S.rlen, S.col,
+                       (const VT*)S.val, x, op);
+  else
+    hipLaunchKernelGGL((k_bsell<B, VT, XT, Acc, Op>), dim3(grid_for(S.nslices * 64)), dim3(kBlock),
+                       0, ctx->stream, S.nslices, S.sptr, S.row, S.rlen, S.col, (const VT*)S.val,
+                       x, op);
 }
 
 template <int B, typename XT, typename Acc, class Op>
@@ -1301,6 +1306,7 @@ int bsell_build(gh_ctx* ctx, int64_t n, int B, const int32_t* rowptr, const int3
       for (int32_t q = rowptr[i]; q < rowptr[i + 1]; ++q) c += kept(q, r);
       if (c > 65535) return fail(GH_EINVAL, "block row %lld has more than 65535 entries", (long long)i);
       len[i * B + r] = (uint16_t)c;
+      S->width = std::max<int>(S->width, (int)c);
       stored += c;
     }
   // longest rows first inside each window, so that slices hold rows of equal length
@@ -2079,6 +2085,12 @@ int gh_csr_layout(const gh_csr* A, int64_t* out) {
 }
 
 int64_t gh_csr_shared_entries(const gh_csr* A) { return A ? A->sell.shared : 0; }
+
+int gh_csr_waves(const gh_csr* A) {
+  if (!A || A->host_only) return 0;
+  if (A->ncomp == 1) return std::max(sell_fold_waves(A->sell), 1);
+  return A->bsell.B && bsell_is_split(A->bsell) ? kBSplit : 1;
+}
 
 static int vec_matches(const gh_csr* A, const gh_vec* v) {
   return v && v->n == A->n && v->ncomp == A->ncomp;

@@ -172,6 +172,7 @@ struct BSell {
   int64_t nslices = 0;
   int64_t slots = 0;      // padded entries (multiple of 64)
   int64_t stored = 0;     // entries kept
+  int width = 0;          // entries of the longest component row
   uint32_t* sptr = nullptr;  // nslices+1, in units of 64 entries
   int32_t* row = nullptr;    // nslices*64 component row of each lane (-1: none)
   uint16_t* rlen = nullptr;  // nslices*64 entries of each lane

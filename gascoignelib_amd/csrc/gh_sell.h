@@ -166,20 +166,83 @@ __device__ __forceinline__ void load_block_row(const T* __restrict__ p, Acc (&o)
 // the row's column order) sum = sum_c A(r, c) x_c from zero, then
 // acc = op.step(acc, sum) -- the per-block sums of k_bsr, in the same order,
 // so both kernels return the same bits.  Only all-zero block rows are left
-// out (their sum is an exact zero).  One wavefront per slice would be bound by
-// the chain column -> x block of its rows (up to 125 entries for a Stokes-LPS
-// pressure row), so a workgroup of kBSplit wavefronts takes a slice: they form
-// the per-block sums of kBSplit * kBEntries entries of the 64 rows at a time,
-// side by side, into LDS, and wavefront 0 folds them into the rows in entry
-// order.  Entries past a row's end exist in the padded slice (column 0) and are
+// out (their sum is an exact zero).
+template <int B, typename VT, typename XT, typename Acc, class Op>
+__global__ __launch_bounds__(kBlock) void k_bsell(int64_t nslices, const uint32_t* __restrict__ sptr,
+                                                  const int32_t* __restrict__ row,
+                                                  const uint16_t* __restrict__ rlen,
+                                                  const int32_t* __restrict__ col,
+                                                  const VT* __restrict__ val,
+                                                  const XT* __restrict__ x, Op op) {
+  const int64_t g = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  const int64_t s = g >> 6;
+  if (s >= nslices) return;
+  const int32_t t = row[g];
+  if (t < 0) return;
+  const int len = rlen[g];
+  const int64_t p0 = (int64_t)sptr[s] * 64 + (threadIdx.x & 63);
+  Acc acc = op.init(t);
+  const int lane = threadIdx.x & 63;
+  const int64_t v0 = (int64_t)sptr[s] * B * 64 + lane;  // value c of entry k: v0 + (k*B + c)*64
+  int k = 0;
+  // Four entries per step.  The step's value and x loads are all issued
+  // before its arithmetic (the scheduling barrier keeps the compiler from
+  // serialising the x gathers to save registers), and the next step's columns
+  // are fetched one step ahead.
+  int32_t c[4];
+  if (len >= 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = col[p0 + (int64_t)u * 64];
+  }
+  for (; k + 4 <= len; k += 4) {
+    Acc m[4][B], q[4][B];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int cc = 0; cc < B; ++cc) m[u][cc] = (Acc)ld(val + v0 + ((int64_t)(k + u) * B + cc) * 64);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_block_row<B>(x + (int64_t)c[u] * B, q[u]);
+    if (k + 8 <= len) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = col[p0 + (int64_t)(k + 4 + u) * 64];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      Acc sum = (Acc)0;
+#pragma unroll
+      for (int cc = 0; cc < B; ++cc) sum = add_rn(sum, mul_rn(m[u][cc], q[u][cc]));
+      acc = op.step(acc, sum);
+    }
+  }
+  for (; k < len; ++k) {
+    Acc m[B], q[B];
+#pragma unroll
+    for (int cc = 0; cc < B; ++cc) m[cc] = (Acc)ld(val + v0 + ((int64_t)k * B + cc) * 64);
+    load_block_row<B>(x + (int64_t)col[p0 + (int64_t)k * 64] * B, q);
+    Acc sum = (Acc)0;
+#pragma unroll
+    for (int cc = 0; cc < B; ++cc) sum = add_rn(sum, mul_rn(m[cc], q[cc]));
+    acc = op.step(acc, sum);
+  }
+  op.finish(t, acc);
+}
+
+// k_bsell where one wavefront per slice is bound by the chain column -> x block
+// of its longest rows (125 entries for a Stokes-LPS pressure row): a workgroup of
+// kBSplit wavefronts takes a slice.  They form the per-block sums of kBSplit *
+// kBEntries entries of the 64 rows at a time, side by side, into LDS, and
+// wavefront 0 folds them into the rows in entry order.  Entry k of a round goes to
+// wavefront k % kBSplit, so that the last, partial round is as short for each of
+// them.  Entries past a row's end exist in the padded slice (column 0) and are
 // formed but not folded.  Two buffers, one barrier per round.  Stokes-LPS
-// residuals against one wavefront per slice: 32^3 80 -> 35 us in FP64 (134 MB,
-// 3.8 TB/s), 36 -> 21 in FP32; 64^3 325 -> 290 and 186 -> 146 (4.2 TB/s); 4913
-// nodes 27 -> 13 and 13 -> 10.5, launch and copy latency included.
+// residuals against k_bsell: 32^3 79 -> 33 us in FP64 (134 MB, 4.1 TB/s), 36 -> 22
+// in FP32; 64^3 330 -> 251 (1.12 GB, 4.5 TB/s) and 182 -> 135; 4913 nodes 26 -> 13
+// and 13 -> 10.4, launch and copy latency included.
 constexpr int kBSplit = 4;
 constexpr int kBEntries = 8;
 template <int B, typename VT, typename XT, typename Acc, class Op>
-__global__ __launch_bounds__(64 * kBSplit) void k_bsell(
+__global__ __launch_bounds__(64 * kBSplit) void k_bsell_split(
     const uint32_t* __restrict__ sptr, const int32_t* __restrict__ row,
     const uint16_t* __restrict__ rlen, const int32_t* __restrict__ col,
     const VT* __restrict__ val, const XT* __restrict__ x, Op op) {
@@ -196,39 +259,41 @@ __global__ __launch_bounds__(64 * kBSplit) void k_bsell(
   const VT* vp = val + s0 * B * 64 + lane;
   Acc acc = (Acc)0;
   if (w == 0 && t >= 0) acc = op.init(t);
-  for (int c0 = 0, buf = 0; c0 < width; c0 += C, buf ^= 1) {
-    const int k0 = c0 + w * kBEntries;
-    Acc m[kBEntries][B], q[kBEntries][B];
-    int32_t c[kBEntries];
-    // (the conditions are the same for the whole wavefront)
-    if (k0 + kBEntries <= width) {
+  // E entries from c0 on, every kBSplit-th from the wavefront's own; those past
+  // the slice's width repeat its last one
+  auto batch = [&](auto num, int c0, int buf) {
+    constexpr int E = decltype(num)::value;
+    Acc m[E][B], q[E][B];
+    int32_t c[E];
+    int64_t k[E];
 #pragma unroll
-      for (int u = 0; u < kBEntries; ++u) c[u] = cp[(int64_t)(k0 + u) * 64];
+    for (int u = 0; u < E; ++u) k[u] = min(c0 + u * kBSplit + w, width - 1);
 #pragma unroll
-      for (int u = 0; u < kBEntries; ++u)
+    for (int u = 0; u < E; ++u) c[u] = cp[k[u] * 64];
 #pragma unroll
-        for (int cc = 0; cc < B; ++cc)
-          m[u][cc] = (Acc)ld(vp + ((int64_t)(k0 + u) * B + cc) * 64);
+    for (int u = 0; u < E; ++u)
 #pragma unroll
-      for (int u = 0; u < kBEntries; ++u) load_block_row<B>(x + (int64_t)c[u] * B, q[u]);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int cc = 0; cc < B; ++cc) m[u][cc] = (Acc)ld(vp + (k[u] * B + cc) * 64);
 #pragma unroll
-      for (int u = 0; u < kBEntries; ++u) {
-        Acc sum = (Acc)0;
+    for (int u = 0; u < E; ++u) load_block_row<B>(x + (int64_t)c[u] * B, q[u]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int cc = 0; cc < B; ++cc) sum = add_rn(sum, mul_rn(m[u][cc], q[u][cc]));
-        part[buf][w * kBEntries + u][lane] = sum;
-      }
-    } else {
-      for (int u = 0; u < kBEntries && k0 + u < width; ++u) {
-        load_block_row<B>(x + (int64_t)cp[(int64_t)(k0 + u) * 64] * B, q[0]);
-        Acc sum = (Acc)0;
+    for (int u = 0; u < E; ++u) {
+      Acc sum = (Acc)0;
 #pragma unroll
-        for (int cc = 0; cc < B; ++cc)
-          sum = add_rn(sum, mul_rn((Acc)ld(vp + ((int64_t)(k0 + u) * B + cc) * 64), q[0][cc]));
-        part[buf][w * kBEntries + u][lane] = sum;
-      }
+      for (int cc = 0; cc < B; ++cc) sum = add_rn(sum, mul_rn(m[u][cc], q[u][cc]));
+      part[buf][u * kBSplit + w][lane] = sum;
     }
+  };
+  for (int c0 = 0, buf = 0; c0 < width; c0 += C, buf ^= 1) {
+    // (the conditions are the same for the whole wavefront)
+    const int left = width - c0 - w;
+    if (left > 4 * kBSplit)
+      batch(std::integral_constant<int, kBEntries>{}, c0, buf);
+    else if (left > kBSplit)
+      batch(std::integral_constant<int, 4>{}, c0, buf);
+    else if (left > 0)
+      batch(std::integral_constant<int, 1>{}, c0, buf);
     __syncthreads();
     if (w == 0) {
       const int n = min(C, width - c0);
@@ -240,6 +305,23 @@ __global__ __launch_bounds__(64 * kBSplit) void k_bsell(
     }
   }
   if (w == 0 && t >= 0) op.finish(t, acc);
+}
+
+// Which of the two runs.  The split pays where the chain of the longest rows is
+// longer than the sweep's share of the chip takes: with few slices (2 per CU;
+// 27-entry rows, B = 4, 500 slices 9.8 -> 6.5 us in FP64 and 5.1 -> 4.6 in FP32,
+// 125 slices 7.4 -> 4.9 and 5.0 -> 3.9), and where a few long rows hold most of the
+// entries (Stokes-LPS).  Otherwise the slices fill the chip one wavefront each, and
+// LDS and barriers only cost: 9-entry rows (2D), 263 K nodes, B = 2 17 -> 25 us,
+// B = 4 70 -> 94; 27-entry rows, 275 K nodes, B = 2 50 -> 58; 36 entries, 1000
+// slices, B = 4 14.7 -> 16.7; 96 entries for every row, 2000 slices 36 -> 38.  Rows
+// of up to 18 entries have too short a chain (13 entries, 16 slices 3.6 -> 3.9 us).
+constexpr int kBSplitRow = 24, kBSplitLong = 64;
+constexpr int64_t kBSplitSlices = 512;
+inline bool bsell_is_split(const BSell& S) {
+  if (S.width < kBSplitRow) return false;
+  if (S.nslices <= kBSplitSlices) return true;
+  return S.width > kBSplitLong && S.nslices * (int64_t)S.width * 64 >= 2 * S.slots;
 }
 
 // One row of a valued operator: entries k = 0..len-1 at stride kSlice, column

@@ -98,6 +98,7 @@ HIP_SIGNATURES = {
     "gh_csr_prec": (C.c_int, [vp]),
     "gh_csr_layout": (C.c_int, [vp, i64p]),
     "gh_csr_shared_entries": (C.c_int64, [vp]),
+    "gh_csr_waves": (C.c_int, [vp]),
     "gh_spmv": (C.c_int, [vp, vp, vp, vp, C.c_double, C.c_double]),
     "gh_spmv_t": (C.c_int, [vp, vp, vp, vp, C.c_double, C.c_double]),
     "gh_residual": (C.c_int, [vp, vp, vp, vp, vp]),

@@ -137,6 +137,9 @@ int gh_csr_layout(const gh_csr* A, int64_t* out);
 /* stored entries whose values a sweep takes from rows shared by whole slices
  * (a slice whose 64 rows hold equal values stores them, but does not read them) */
 int64_t gh_csr_shared_entries(const gh_csr* A);
+/* wavefronts that share a slice of 64 rows in products of FP64 vectors: 1, 4
+ * or 8 (the results are the same, bit for bit); 0 without a device layout */
+int gh_csr_waves(const gh_csr* A);
 /* The values the device holds, in A's CSR order (nnz*B*B, reduced-precision
  * values widened to FP64); the D2H half of operator<< (print of the device
  * matrix, cuda/cudacsrmatrixinterface.cc:439).  Synchronises. */

@@ -163,6 +163,58 @@ def test_block_products_bitexact(ctx, B):
     assert np.abs(Y32.copy_back() - ye).max() <= 1e-5 * np.abs(ye).max()
 
 
+def band_blocks(n, B, wide, narrow, seed):
+    """Block rows of `wide` blocks around the diagonal whose last component row
+    fills every block; the other component rows fill the first `narrow` of them
+    and the diagonal one, the rest is zero."""
+    r = np.random.default_rng(seed)
+    cols = np.sort((np.arange(n)[:, None] + np.arange(wide) * 3) % n, axis=1)
+    # multiples of 2^-10, exact in f16
+    val = r.integers(1, 1025, (n, wide, B, B)) * r.choice([-1.0, 1.0], (n, wide, B, B)) / 1024
+    val[:, narrow:, :B - 1] = 0.0
+    val[cols == np.arange(n)[:, None]] = np.eye(B) * (B * wide + 1.0)
+    return ((np.arange(n + 1) * wide).astype(np.int32), cols.reshape(-1).astype(np.int32),
+            val.reshape(-1))
+
+
+# 4 wavefronts share a slice where it is one of up to 512 with rows of 24 entries
+# or more, or where rows of more than 64 are twice the mean; around the rounds of
+# 32 entries and their partial batches of 4, 16 and 32
+@pytest.mark.parametrize("n,B,wide,narrow,waves", [
+    (700, 2, 9, 9, 1), (700, 3, 23, 23, 1), (700, 4, 24, 24, 4), (700, 2, 31, 31, 4),
+    (700, 3, 32, 32, 4), (700, 4, 33, 33, 4), (190, 2, 36, 5, 4), (700, 3, 48, 48, 4),
+    (700, 4, 49, 20, 4), (700, 2, 70, 70, 4), (8192, 4, 27, 27, 4), (8193, 4, 27, 27, 1),
+    (9000, 4, 64, 8, 1), (9000, 4, 70, 8, 4), (9000, 4, 70, 70, 1), (17000, 2, 100, 3, 1),
+    (17000, 3, 100, 3, 4), (1, 4, 1, 1, 1)])
+def test_block_products_forms(ctx, n, B, wide, narrow, waves):
+    """FP64 block products keep the oracle's bits in both forms, and each size
+    takes the form that is faster for it."""
+    print(f"[block forms n={n} B={B} {wide}/{narrow}]", flush=True)
+    rowptr, col, val = band_blocks(n, B, wide, narrow, n + wide)
+    A = H.CudaCSRMatrixInterface(ctx, rowptr, col, val, B)
+    assert A.layout()["waves"] == waves
+    Ao = O.Matrix(rowptr, col, val, B)
+    r = np.random.default_rng(wide)
+    x, b = r.uniform(-1, 1, n * B), r.uniform(-1, 1, n * B)
+    X = H.CudaVectorInterface.from_global(ctx, x, B)
+    R = H.CudaVectorInterface(ctx, n, B)
+    A.residual(R, X, H.CudaVectorInterface.from_global(ctx, b, B))
+    ro = np.zeros(n * B)
+    Ao.residual(ro, x, b)
+    assert np.array_equal(R.copy_back(), ro)
+    # |computed - exact| <= (terms + conversions of x and b + the difference) 2^-24
+    # times the sum of the terms' absolute values
+    bound = np.abs(val).reshape(n, wide, B, B)
+    xs = np.abs(x).reshape(n, B)[col.reshape(n, wide)]
+    bound = np.einsum("nwrc,nwc->nr", bound, xs).reshape(-1) + np.abs(b)
+    for prec in ("f32", "f16"):
+        A32 = H.CudaCSRMatrixInterface(ctx, rowptr, col, val, B, prec)
+        X32, B32 = (H.CudaVectorInterface.from_global(ctx, v, B, "f32") for v in (x, b))
+        R32 = H.CudaVectorInterface(ctx, n, B, "f32")
+        A32.residual(R32, X32, B32)
+        assert np.all(np.abs(R32.copy_back() - ro) <= 2.0 ** -24 * (B * wide + 4) * bound), prec
+
+
 def test_block_transpose_product(ctx, h8):
     """y = d A^T x + b y for the 4x4-block operator against scipy"""
     import scipy.sparse as sp
