@@ -1051,12 +1051,14 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
   uint64_t units = 0;
   S->narrow = 0;
   S->patterned = 0;
+  S->single = 0;
   S->col_bytes = 0;
   for (int64_t s = 0; s < ns; ++s) {
     if (pat[s]) {
       cptr[s] = 0x40000000u;
       S->patterned++;
       if (one[s]) {  // one pattern for the whole wavefront: its id in cbase
+        S->single += sptr[s + 1] - sptr[s];
         cptr[s] |= 0x20000000u;
         cbase[s] = (uint32_t)rpid[s * kSlice];
       }
@@ -1092,7 +1094,7 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
         const int lane = (int)(j % kSlice);
         const int64_t i = s * kSlice + lane;
         const bool used = i < n && (int64_t)(j / kSlice) < rlen[i];
-        const uint32_t c = used ? scol[sptr[s] + j] : cbase[s];  // padding: never read
+        const uint32_t c = used ? scol[sptr[s] + j] : cbase[s];  // padding: a valid column
         if (wide[s]) {
           cidx[at + 2 * j] = (uint16_t)(c & 0xFFFFu);
           cidx[at + 2 * j + 1] = (uint16_t)(c >> 16);

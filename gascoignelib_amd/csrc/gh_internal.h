@@ -128,7 +128,9 @@ struct Sell {
   //     rlen[row] holds its id, columns are row + ptab[pstart[id] + k]; with
   //     bit 29 all 64 rows share one pattern, whose id is cbase[s];
   //   16-bit offsets from cbase[s] (cptr = start in 16-bit units);
-  //   32-bit indices (cptr bit 31, start in 16-bit units, 4-byte aligned)
+  //   32-bit indices (cptr bit 31, start in 16-bit units, 4-byte aligned).
+  // Padding (entries past a row's end, lanes past the last row) holds a valid
+  // column: k_sell_fold gathers x through it and drops the product.
   uint16_t* cidx = nullptr;
   uint32_t* cptr = nullptr;
   uint32_t* cbase = nullptr;
@@ -147,6 +149,7 @@ struct Sell {
   int64_t nvtab = 0;
   int64_t shared = 0;        // stored entries whose values come from vtab
   int64_t patterned = 0;     // slices in pattern mode
+  int64_t single = 0;        // slots of the slices whose rows share one pattern
   int64_t col_bytes = 0;     // column bytes a sweep reads (stored entries only)
   // row run by each slot (valued operators whose rows were grouped by
   // pattern; nullptr: slot = row); rlen and the slot arrays are in slot order

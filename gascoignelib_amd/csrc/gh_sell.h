@@ -663,18 +663,32 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_fold(
   if (w == 0 && active) op.finish(row, acc);
 }
 
-// Wavefronts per slice of an exact sweep (0: k_sell).  The fold pays where rows
-// are long; rows of up to 27 entries (Q1) are faster in k_sell from 117 K rows up
-// (7.8 against 10.1 us) and equal below.  Two rounds of 64 entries keep few
-// slices busier than four of 32, which leave LDS for more slices per CU: FP64
-// residuals of Q2 rows (62 entries on average, 125 to 285 at most), k_sell / 4 / 8
-// wavefronts: 729 rows 8.3 / 6.7 / 5.4 us, 14 K 17.5 / 11.7 / 9.0, 79 K 38 / 27 /
-// 24, 275 K 60 / 45 / 56, 352 K 109 / 64 / 78.
-constexpr int kFoldRow = 32;
-constexpr int64_t kFoldFewSlices = 2048;
+// Wavefronts per slice of an exact sweep (0: k_sell).  The fold pays where the
+// chains of long rows bound the sweep, FP64 residuals, k_sell / 4 / 8 wavefronts:
+//  * Few slices: 8 wavefronts take 64 entries per round, their 64 KB of LDS leave a
+//    CU two workgroups; 4 take 32 and leave five.  The longer the rows, the more
+//    rounds 8 save and the more slices that pays for.  Q2 (125 to 285 entries at
+//    most), 12 slices 8.3 / 6.5 / 5.4 us, 562 slices 13.1 / 10.7 / 10.0, 1231 slices
+//    39 / 25.4 / 24.0; rows of 48, 125 slices 5.4 / 4.2 / 4.0, 469 slices 5.7 / 4.7 /
+//    5.3; of 96, 469 slices 9.2 / 6.2 / 6.8; of 51 (Q1 with hanging nodes, mean 18),
+//    342 slices 6.4 / 5.1 / 5.6.
+//  * Many slices: only where rows of more than 64 entries are well above the mean,
+//    so that few wavefronts of k_sell would hold most of the entries.  Q2, 275 K
+//    rows 60 / 44 / 54, 352 K 109 / 60 / 75.  Rows of 27 and up to 51 entries lose:
+//    532 K adaptive Q1 rows 25 / 36 / 67; rows of 27 and 48, 60 K 6.2 / 6.9 / 8.7.  So
+//    do equal rows: 96 entries each, 120 K 22.7 / 24.6 / 30.1.
+//  * Single-pattern slices take their columns from scalar registers, k_sell's loads
+//    then wait for nothing: rows of 27 and 96, 120 K rows 14.3 / 17.3 / 23.0 against
+//    19.2 / 17.6 / 23.0 with columns in memory.  Where they hold most of the entries,
+//    the fold is for few slices only.
+constexpr int kFoldRow = 32, kFoldLong = 64;
+constexpr int64_t kFoldSlices4 = 512;
 inline int sell_fold_waves(const Sell& S) {
   if (S.maxlen <= kFoldRow) return 0;
-  return S.nslices <= kFoldFewSlices ? 8 : 4;
+  if (S.nslices <= 5 * (int64_t)S.maxlen) return 8;
+  if (2 * S.single > S.slots) return 0;
+  if (S.nslices <= kFoldSlices4) return 4;
+  return S.maxlen > kFoldLong && 2 * S.nslices * S.maxlen * kSlice >= 3 * S.slots ? 4 : 0;
 }
 
 // Split factor of a reduced-precision sweep: double K while the level runs

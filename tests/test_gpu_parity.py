@@ -667,13 +667,51 @@ def test_shared_values(ctx, kind, refine):
 @pytest.mark.parametrize("n,L", [(90, 33), (700, 40), (5000, 64), (700, 66), (5000, 100), (90, 128),
                                  (700, 130), (700, 300), (70000, 50), (132000, 36)])
 def test_fp64_sweeps_long_rows_bitexact(ctx, n, L):
-    """Rows longer than the 32 entries from which FP64 sweeps form their
+    """Rows longer than the 32 entries from which FP64 sweeps may form their
     products on 4 or 8 wavefronts per slice and fold them in entry order:
     around the rounds of 32 and 64 entries, partial last slices, every column
-    encoding, 8 wavefronts (up to 2048 slices) and 4: the oracle's bits."""
+    encoding: the oracle's bits."""
     print(f"[n={n} L={L}]", flush=True)
     rowptr, col, val = long_row_matrix(n, L, seed=3 * L + n)
     A = H.CudaCSRMatrixInterface(ctx, rowptr, col, val)
+    check_products_vs_oracle(ctx, A, rowptr, col, val, L)
+
+
+def mixed_rows(n, L, share, short, columns, seed):
+    """runs of 64 rows, a share of them with L entries and the others with `short`:
+    bands of one pattern, or random columns"""
+    rng = np.random.default_rng(seed)
+    runs = (n + 63) // 64
+    lens = np.repeat(np.where(np.arange(runs) % 20 < round(20 * share), L, short), 64)[:n]
+    i = np.repeat(np.arange(n), lens)
+    k = np.arange(len(i)) - np.repeat(np.cumsum(lens) - lens, lens)
+    if columns == "band":
+        col = np.clip(i + 3 * (k - np.repeat(lens // 2, lens)), 0, n - 1)
+    else:
+        col = rng.integers(0, n, len(i))
+    A = sp.coo_matrix((np.r_[rng.uniform(0.5, 1, len(i)), np.full(n, L + 1.0)],
+                       (np.r_[i, np.arange(n)], np.r_[col, np.arange(n)])), (n, n)).tocsr()
+    A.sum_duplicates()
+    return A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data
+
+
+# few slices (5 per entry of the longest row) take 8 wavefronts, up to 512 take 4;
+# more only where rows of more than 64 entries are 1.5 times the mean and most
+# entries lie outside single-pattern slices
+@pytest.mark.parametrize("n,L,share,short,columns,waves", [
+    (640, 32, 1.0, 32, "random", 8), (640, 31, 1.0, 31, "random", 1),
+    (5000, 40, 1.0, 40, "band", 8), (10000, 33, 0.5, 9, "random", 8),
+    (12000, 36, 0.1, 27, "random", 4), (12000, 36, 1.0, 36, "band", 1),
+    (32768, 60, 0.5, 27, "random", 4), (32769, 60, 0.5, 27, "random", 1),
+    (50000, 51, 0.05, 18, "random", 1), (50000, 100, 0.25, 9, "random", 4),
+    (50000, 100, 0.25, 9, "band", 1), (50000, 100, 1.0, 100, "random", 1)])
+def test_fp64_sweep_forms(ctx, n, L, share, short, columns, waves):
+    """each matrix takes the form of the FP64 sweep that is faster for it, and
+    every form keeps the oracle's bits"""
+    print(f"[sweep form n={n} L={L} {share} {short} {columns}]", flush=True)
+    rowptr, col, val = mixed_rows(n, L, share, short, columns, L + n)
+    A = H.CudaCSRMatrixInterface(ctx, rowptr, col, val)
+    assert A.layout()["waves"] == waves
     check_products_vs_oracle(ctx, A, rowptr, col, val, L)
 
 
