@@ -37,6 +37,7 @@ namespace gh {
 struct IluSlices {
   int64_t nslices = 0, nentries = 0;
   std::vector<int64_t> lslice;  // level L covers slices [lslice[L], lslice[L+1]) (host)
+  std::vector<int32_t> lwidth;  // entries of level L's longest row (host)
   int32_t* row = nullptr;       // nslices*64 ILU rows, -1 in padding
   int32_t* len = nullptr;       // nslices*64 entry counts
   int64_t* base = nullptr;      // nslices + 1 first entries
@@ -241,14 +242,12 @@ __global__ __launch_bounds__(kBlock) void k_ilu_sweep(int64_t s0, int64_t s1,
 // entries and one per remaining entry.  Entries past a row's end read the row's
 // own y (written only after the last round) and are replaced by +0, which
 // a - 0 leaves as it is.
-// Levels of up to kFoldSlices slices run it: a solve in 8 + 8 colour levels takes
-// 76 us against 94 in FP64 on 65^3 nodes (540 slices a level; FP32 63 against
-// 90), 53 against 75 on 33^3, where the 16 launches are 51; on 129^3 (4200
-// slices) the slices fill the chip by themselves: 328 against 271 (FP32 199, 204).
-constexpr int64_t kFoldSlices = 2048;
 constexpr int kFoldWaves = 4;
 constexpr int kFoldEntries = 8;
 constexpr int kFoldRound = kFoldWaves * kFoldEntries;
+// Against k_ilu_sweep a solve in 8 + 8 colour levels takes 77 us instead of 90 in
+// FP64 on 65^3 nodes (540 slices a level; FP32 63 instead of 83), 56 instead of 70
+// on 33^3, where the 16 launches are 51.
 template <typename T, typename VT, bool kUpper>
 __global__ __launch_bounds__(64 * kFoldWaves) void k_ilu_fold(
     int64_t s0, const int32_t* __restrict__ row, const int32_t* __restrict__ len,
@@ -318,6 +317,20 @@ __global__ __launch_bounds__(64 * kFoldWaves) void k_ilu_fold(
   }
 }
 
+// Whether a level of `slices` slices, rows of up to `width` entries, runs it: while
+// the slices do not fill the chip by themselves.  In FP64 the 32 KB of LDS leave a
+// CU 5 slices: 73^3 nodes (760 slices a level) 98 -> 81 us, 77^3 (892) 97 -> 88,
+// 81^3 (1038) 101 -> 103, 97^3 (1783) 148 -> 164; rows that k_ilu_sweep takes in one
+// batch of 8 (2D) gain nothing and lose sooner: 301^2 nodes (354) 30.6 -> 29.7,
+// 385^2 (579) 32.0 -> 36.2, 513^2 (1028) 39 -> 46.  In FP32 it is 16 KB and 8 slices:
+// 97^3 103 -> 91, 101^3 (2013) 107 -> 98, 705^2 (1942) 41 -> 38; 129^3 (4193) 204 -> 199.
+constexpr int kFoldNarrow = 8;
+constexpr int64_t kFoldSlicesNarrow64 = 512, kFoldSlices64 = 960, kFoldSlices32 = 2048;
+bool fold_pays(int64_t slices, int32_t width, bool fp64) {
+  if (!fp64) return slices <= kFoldSlices32;
+  return slices <= (width > kFoldNarrow ? kFoldSlices64 : kFoldSlicesNarrow64);
+}
+
 // sliced values (and the diagonal inverses) from the CSR factors
 __global__ __launch_bounds__(kBlock) void k_ilu_fill(int64_t m, int BB, const int32_t* __restrict__ map,
                                                      const double* __restrict__ val,
@@ -355,7 +368,7 @@ int solve_levels(gh_ctx* ctx, const gh_ilu* I, bool fp64, const T* xin, T* y, T*
       const int64_t s0 = S.lslice[L], s1 = S.lslice[L + 1];
       const unsigned g = (unsigned)((s1 - s0 + kBlock / 64 - 1) / (kBlock / 64));
       if constexpr (B == 1) {
-        if (s1 > s0 && s1 - s0 <= kFoldSlices) {
+        if (s1 > s0 && fold_pays(s1 - s0, S.lwidth[L], std::is_same<T, double>::value)) {
           const dim3 gf((unsigned)(s1 - s0)), tf(64 * kFoldWaves);
           if (part == 0)
             hipLaunchKernelGGL((k_ilu_fold<T, VT, false>), gf, tf, 0, ctx->stream, s0, S.row, S.len,
@@ -438,6 +451,10 @@ int build_slices(gh_ctx* ctx, const std::vector<int32_t>& rows, const std::vecto
     for (int l = 0; l < 64; ++l) w = std::max(w, hlen[sl * 64 + l]);
     hbase[sl + 1] = hbase[sl] + (int64_t)w * 64;
   }
+  S->lwidth.assign(nl, 0);
+  for (size_t L = 0; L < nl; ++L)
+    for (int64_t sl = S->lslice[L]; sl < S->lslice[L + 1]; ++sl)
+      S->lwidth[L] = std::max(S->lwidth[L], (int32_t)((hbase[sl + 1] - hbase[sl]) / 64));
   const int64_t ne = hbase[ns];
   std::vector<int32_t> hcol(ne, 0), hmap(ne, -1);
   for (int64_t sl = 0; sl < ns; ++sl)
@@ -608,6 +625,17 @@ int gh_ilu_levels(const gh_ilu* I, int32_t* forward, int32_t* backward) {
   *forward = (int32_t)I->lptr_f.size() - 1;
   *backward = (int32_t)I->lptr_b.size() - 1;
   return GH_OK;
+}
+
+int32_t gh_ilu_split_levels(const gh_ilu* I, int prec) {
+  if (!I || I->B != 1) return 0;
+  int32_t k = 0;
+  for (const IluSlices* S : {&I->lo, &I->up})
+    for (size_t L = 0; L < S->lwidth.size(); ++L) {
+      const int64_t slices = S->lslice[L + 1] - S->lslice[L];
+      k += slices > 0 && fold_pays(slices, S->lwidth[L], prec == GH_F64);
+    }
+  return k;
 }
 
 int gh_ilu_download(gh_ctx* ctx, const gh_ilu* I, int32_t* rowptr, int32_t* col, int32_t* diag,

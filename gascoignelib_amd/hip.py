@@ -658,6 +658,11 @@ class SparseBlockIlu:
         check(N.hip().gh_ilu_levels(self.h, C.byref(f), C.byref(b)))
         return f.value, b.value
 
+    def split_levels(self, prec="f64"):
+        """levels of both triangles that a solve of a `prec` vector runs with 4
+        wavefronts per slice of 64 rows"""
+        return int(N.hip().gh_ilu_split_levels(self.h, N.PREC[prec]))
+
     def factors(self, nnz):
         """(rowptr, col, diag, val) of the factors in ILU numbering."""
         B = self.ncomp

@@ -148,6 +148,7 @@ HIP_SIGNATURES = {
     "gh_ilu_destroy": (C.c_int, [vp]),
     "gh_ilu_solve": (C.c_int, [vp, vp, vp]),
     "gh_ilu_levels": (C.c_int, [vp, i32p, i32p]),
+    "gh_ilu_split_levels": (C.c_int32, [vp, C.c_int]),
     "gh_ilu_download": (C.c_int, [vp, vp, i32p, i32p, i32p, f64p]),
     "gh_mg_set_ilu": (C.c_int, [vp, C.c_int, i32p]),
     "gh_patches_create": (C.c_int, [vp, C.c_int, C.c_int64, f64p, C.c_int64, i32p, P(vp)]),

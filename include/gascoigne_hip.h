@@ -207,6 +207,9 @@ int gh_ilu_destroy(gh_ilu* I);
 int gh_ilu_solve(gh_ctx* ctx, const gh_ilu* I, gh_vec* x);
 /* Level counts of the forward (lower) and backward (upper) schedules. */
 int gh_ilu_levels(const gh_ilu* I, int32_t* forward, int32_t* backward);
+/* How many of them, in both schedules, a solve of a `prec` vector runs with 4
+ * wavefronts per slice of 64 rows (the results are the same). */
+int32_t gh_ilu_split_levels(const gh_ilu* I, int prec);
 /* The factors in ILU numbering (n+1 rowptr, nnz col, n diagonal positions,
  * nnz*B*B values, row-major blocks); any pointer may be NULL. */
 int gh_ilu_download(gh_ctx* ctx, const gh_ilu* I, int32_t* rowptr, int32_t* col, int32_t* diag,

@@ -156,6 +156,37 @@ def test_scalar_ilu_shapes(ctx, n, offsets, order):
     assert np.abs(X32.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
 
 
+# two levels per triangle, of rows without entries and rows of k; 4 wavefronts per
+# slice up to 2048 slices in FP32 and up to 512 in FP64, 960 for rows of more
+# than the 8 entries that one wavefront takes in a batch
+@pytest.mark.parametrize("slices,k,split64,split32", [
+    (1, 1, 4, 4), (512, 8, 4, 4), (513, 8, 0, 4), (512, 9, 4, 4), (513, 9, 2, 4), (960, 9, 2, 4),
+    (961, 9, 0, 4), (961, 33, 0, 4), (300, 33, 4, 4), (2048, 1, 0, 4), (2049, 1, 0, 0)])
+def test_ilu_level_forms(ctx, slices, k, split64, split32):
+    print(f"[ilu slices={slices} k={k}]", flush=True)
+    m = 64 * slices - 3 * (slices > 1)  # a partial last slice
+    half = np.sort((np.arange(m)[:, None] + 7 * np.arange(k)) % m, axis=1)
+    rows = np.arange(2 * m)[:, None]
+    col = np.sort(np.concatenate([np.concatenate([half + m, half]), rows], axis=1), axis=1)
+    r = np.random.default_rng(slices + k)
+    val = r.uniform(-1, 1, col.shape)
+    val[col == rows] = k + 2.0
+    rp = (np.arange(2 * m + 1) * (k + 1)).astype(np.int32)
+    col, val = col.reshape(-1).astype(np.int32), val.reshape(-1)
+    I = H.SparseBlockIlu(ctx, H.CudaCSRMatrixInterface(ctx, rp, col, val))
+    assert I.levels() == (2, 2)
+    assert (I.split_levels("f64"), I.split_levels("f32")) == (split64, split32)
+    x = r.uniform(-1, 1, 2 * m)
+    xo = x.copy()
+    O.Ilu(O.Matrix(rp, col, val), None).solve(xo)
+    X = H.CudaVectorInterface.from_global(ctx, x)
+    I.solve(X)
+    assert np.array_equal(X.copy_back(), xo)
+    X32 = H.CudaVectorInterface.from_global(ctx, x, 1, "f32")
+    I.solve(X32)
+    assert np.abs(X32.copy_back() - xo).max() <= 1e-5 * np.abs(xo).max()
+
+
 def test_colour_order_levels_and_solve(ctx):
     """in the colour order each triangle has one level per colour; factors and
     solves still equal the oracle's, and the FP32 solve is close"""
