@@ -57,7 +57,8 @@ constexpr int kTileRows = 32, kTileCols = 64;  // update: entries per workgroup 
 
 // columns k0 .. k0 + w - 1 (w <= kPanel): W (kPanel x m) receives the panel,
 // piv[k0 + t] the pivot rows; taken[row] is k0 + 1 for the rows that got a pivot
-// here.  flag: the first column whose candidates are all zero, plus one.
+// here.  flag: the first column whose candidates are zeros, plus one (NaNs among
+// them are no zeros: the inverse is then NaN, as from an LU).
 // A thread's rows turn by one register per column, so that the column in hand is
 // always a[.][0] and the loop stays small.
 __global__ __launch_bounds__(kGjThreads) void k_gj_panel(int m, int k0, int w,
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(kGjThreads) void k_gj_panel(int m, int k0, int w,
         free_row[g] = false;
         taken[gr] = k0 + 1;
         piv[k0 + t] = gr;
-        if (gb == 0.0) atomicCAS(flag, 0, k0 + t + 1);
+        if (a[g][0] == 0.0) atomicCAS(flag, 0, k0 + t + 1);  // a NaN is no zero
       }
     }
     __syncthreads();

@@ -92,3 +92,18 @@ def test_dense_inverse_sizes(ctx, n):
     r = np.abs(A @ X.copy_back() - b).max()
     norm = lambda M: np.abs(M).sum(axis=1).max()  # noqa: E731
     assert r <= n * 2.0 ** -52 * norm(A) * norm(np.linalg.inv(A)) * np.abs(b).max()
+
+
+def test_nan_in_a_direct_level_is_not_singular(ctx):
+    """A column without any number takes a NaN as its pivot: the inverse is NaN, as
+    an LU's, and no zero pivot is reported."""
+    n = 70  # three panels
+    rng = np.random.default_rng(1)
+    A = rng.normal(size=(n, n)) + n * np.eye(n)
+    A[3, 5] = np.nan
+    lev = Level(n, 1, np.arange(n + 1, dtype=np.int32) * n,
+                np.tile(np.arange(n, dtype=np.int32), n), A.reshape(-1).copy())
+    mg = H.CudaMultiLevelSolver(ctx, Hierarchy([lev], 3, "nan"), ndirect=n + 1, **MGP)
+    X = mg.new_vector()
+    mg.precondition(X, H.CudaVectorInterface.from_global(ctx, np.ones(n)), x_is_zero=True)
+    assert np.isnan(X.copy_back()).any()
