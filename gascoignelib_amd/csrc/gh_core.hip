@@ -670,6 +670,12 @@ struct KeyTable {
 };
 
 // ------------------------------------------------------------ shared values
+constexpr uint32_t kNoShared = 0xFFFFFFFFu;  // vptr of a slice without a vtab row
+
+__device__ __forceinline__ bool same_bits(double a, double b) {
+  return __builtin_bit_cast(uint64_t, a) == __builtin_bit_cast(uint64_t, b);
+}
+
 // hash[s]: of the slice's row of values where all its rows follow one pattern
 // and hold the same stored values (never 0), else 0.  One wavefront per slice;
 // a lane without a row repeats the last row's slot.
@@ -706,9 +712,10 @@ __global__ __launch_bounds__(kBlock) void k_sell_hash(int64_t n, int64_t nslices
   if ((threadIdx.x & 63) == 0) hash[s] = h;
 }
 
-// vtab rows from their slices' first rows
+// vtab rows from the first rows of the slices that stand for them (vrep); one
+// wavefront each
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void k_sell_vtab(int64_t nslices,
+__global__ __launch_bounds__(kBlock) void k_sell_vtab(int64_t nvrep,
                                                       const uint32_t* __restrict__ sptr,
                                                       const uint32_t* __restrict__ cbase,
                                                       const int32_t* __restrict__ pstart,
@@ -716,8 +723,9 @@ __global__ __launch_bounds__(kBlock) void k_sell_vtab(int64_t nslices,
                                                       const int32_t* __restrict__ vrep,
                                                       const VT* __restrict__ val,
                                                       SharedT<VT>* __restrict__ vtab) {
-  const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
-  if (s >= nslices || vptr[s] == 0xFFFFFFFFu || vrep[s] != (int32_t)s) return;
+  const int64_t r = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
+  if (r >= nvrep) return;
+  const int32_t s = vrep[r];
   const int pid = (int)cbase[s];
   const int len = pstart[pid + 1] - pstart[pid];
   for (int k = threadIdx.x & 63; k < len; k += kSlice)
@@ -733,41 +741,17 @@ __global__ __launch_bounds__(kBlock) void k_sell_mark(int64_t n, int64_t nslices
                                                       const uint32_t* __restrict__ vptr,
                                                       const VT* __restrict__ val,
                                                       const SharedT<VT>* __restrict__ vtab,
-                                                      uint32_t* __restrict__ cptr, int* count) {
+                                                      uint32_t* __restrict__ cptr) {
   const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
-  if (s >= nslices || vptr[s] == 0xFFFFFFFFu) return;  // the whole wavefront
+  if (s >= nslices || vptr[s] == kNoShared) return;  // the whole wavefront
   const int rows = min(kSlice, (int)(n - s * kSlice));
   const int lane = min((int)(threadIdx.x & 63), rows - 1);
   const int pid = (int)cbase[s];
   const int len = pstart[pid + 1] - pstart[pid];
   bool same = true;
-  for (int k = 0; k < len && same; ++k) {
-    const double a = (double)ld(val + sptr[s] + (int64_t)k * kSlice + lane);
-    const double b = (double)vtab[vptr[s] + k];
-    same = __ballot(__builtin_bit_cast(uint64_t, a) != __builtin_bit_cast(uint64_t, b)) == 0;
-  }
-  if ((threadIdx.x & 63) == 0) {
-    cptr[s] = 0x60000000u | (same ? kSharedBit | vptr[s] : 0u);
-    if (same) atomicAdd(count, rows * len);
-  }
-}
-
-template <typename VT>
-static int sell_share_as(gh_ctx* ctx, const Sell& S, int* count) {
-  const dim3 g(grid_for(S.nslices, kBlock / kSlice)), b(kBlock);
-  hipLaunchKernelGGL(k_sell_vtab<VT>, g, b, 0, ctx->stream, S.nslices, S.sptr, S.cbase, S.pstart,
-                     S.vptr, S.vrep, (const VT*)S.val, (SharedT<VT>*)S.vtab);
-  hipLaunchKernelGGL(k_sell_mark<VT>, g, b, 0, ctx->stream, S.n, S.nslices, S.sptr, S.cbase,
-                     S.pstart, S.vptr, (const VT*)S.val, (const SharedT<VT>*)S.vtab, S.cptr, count);
-  GH_HIP(hipGetLastError());
-  return GH_OK;
-}
-
-int sell_share(gh_ctx* ctx, const Sell& S, int* count) {
-  if (!S.vtab) return GH_OK;
-  if (S.prec == GH_F64) return sell_share_as<double>(ctx, S, count);
-  if (S.prec == GH_F32) return sell_share_as<float>(ctx, S, count);
-  return sell_share_as<__half>(ctx, S, count);
+  for (int k = 0; k < len && same; ++k)
+    same = __ballot(!same_bits(ld(val + sptr[s] + (int64_t)k * kSlice + lane), vtab[vptr[s] + k])) == 0;
+  if ((threadIdx.x & 63) == 0) cptr[s] = 0x60000000u | (same ? kSharedBit | vptr[s] : 0u);
 }
 
 // Finds the slices that share values when the layout is built: slices of one
@@ -778,13 +762,11 @@ static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& on
   for (int64_t s = 0; s < ns && !any; ++s) any = one[s] != 0;
   if (!any) return GH_OK;
   uint64_t* d_hash = nullptr;
-  int* d_count = nullptr;
-  if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * (ns + 1)) != hipSuccess)
+  if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * ns) != hipSuccess)
     return fail(GH_ENOMEM, "sell_build: allocation failed");
-  d_count = (int*)(d_hash + ns);
   std::vector<uint64_t> hash(ns);
-  std::vector<uint32_t> cb(ns), vptr(ns, 0xFFFFFFFFu);
-  std::vector<int32_t> vrep(ns, -1), ps(S->npat + 1);
+  std::vector<uint32_t> cb(ns), vptr(ns, kNoShared);
+  std::vector<int32_t> vrep, ps(S->npat + 1);
   auto run = [&]() -> int {
     const dim3 g(grid_for(ns, kBlock / kSlice)), b(kBlock);
     if (S->prec == GH_F64)
@@ -797,7 +779,6 @@ static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& on
       hipLaunchKernelGGL(k_sell_hash<__half>, g, b, 0, ctx->stream, S->n, ns, S->sptr, S->cptr,
                          S->cbase, S->pstart, (const __half*)S->val, d_hash);
     GH_HIP(hipGetLastError());
-    GH_HIP(hipMemsetAsync(d_count, 0, sizeof(int), ctx->stream));
     GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
     GH_HIP(hipMemcpyAsync(cb.data(), S->cbase, sizeof(uint32_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
     GH_HIP(hipMemcpyAsync(ps.data(), S->pstart, sizeof(int32_t) * ps.size(), hipMemcpyDeviceToHost,
@@ -815,23 +796,32 @@ static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& on
         if (total + len > (int64_t)kSharedMask) continue;
         vptr[s] = (uint32_t)total;
         total += len;
+        vrep.push_back((int32_t)s);
       } else {
         vptr[s] = vptr[r];
       }
-      vrep[s] = (int32_t)r;
     }
     if (total == 0) return GH_OK;
+    S->nvrep = (int64_t)vrep.size();
     S->nvtab = total;
     if (hipMalloc(&S->vtab, total * (S->prec == GH_F64 ? 8 : 4)) != hipSuccess)
       return fail(GH_ENOMEM, "sell_build: allocation failed");
     GH_TRY(upload(ctx, &S->vptr, vptr.data(), vptr.size()));
     GH_TRY(upload(ctx, &S->vrep, vrep.data(), vrep.size()));
-    GH_TRY(sell_share(ctx, *S, d_count));
-    int c = 0;
-    GH_HIP(hipMemcpyAsync(&c, d_count, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    GH_HIP(hipStreamSynchronize(ctx->stream));
-    S->shared = (uint32_t)c;
-    return GH_OK;
+    auto mark = [&](auto vt) -> int {
+      using VT = decltype(vt);
+      hipLaunchKernelGGL(k_sell_vtab<VT>, dim3(grid_for(S->nvrep, kBlock / kSlice)), b, 0, ctx->stream,
+                         S->nvrep, S->sptr, S->cbase, S->pstart, S->vptr, S->vrep, (const VT*)S->val,
+                         (SharedT<VT>*)S->vtab);
+      hipLaunchKernelGGL(k_sell_mark<VT>, g, b, 0, ctx->stream, S->n, ns, S->sptr, S->cbase, S->pstart,
+                         S->vptr, (const VT*)S->val, (const SharedT<VT>*)S->vtab, S->cptr);
+      GH_HIP(hipGetLastError());
+      GH_HIP(hipStreamSynchronize(ctx->stream));
+      return GH_OK;
+    };
+    if (S->prec == GH_F64) return mark(double{});
+    if (S->prec == GH_F32) return mark(float{});
+    return mark(__half{});
   };
   const int rc = run();
   (void)hipFree(d_hash);
@@ -1270,11 +1260,12 @@ int sell_build(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const uint32_t* co
 void sell_free(Sell* S) {
   for (void* p : {(void*)S->sptr, (void*)S->rlen, (void*)S->col, S->val, (void*)S->cidx,
                   (void*)S->cptr, (void*)S->cbase, (void*)S->ptab, (void*)S->pstart,
-                  (void*)S->perm, S->vtab, (void*)S->vptr, (void*)S->vrep})
+                  (void*)S->perm, S->vtab, (void*)S->vptr, (void*)S->vrep, (void*)S->vsrc})
     if (p) (void)hipFree(p);
   S->vtab = nullptr;
   S->vptr = nullptr;
   S->vrep = nullptr;
+  S->vsrc = nullptr;
   S->perm = nullptr;
   S->ptab = nullptr;
   S->pstart = nullptr;
@@ -1700,16 +1691,23 @@ static int launch_block_inverse(gh_ctx* ctx, int64_t n, int B, const int32_t* di
 // row at a time (coalesced; 4 rows in flight), rank the kept ones by a
 // ballot and stage them in LDS, up to 128 per row (further ones are stored
 // directly); the group then goes out k by k, the 8 rows of one k being 8
-// adjacent slots.
-template <typename VT>
+// adjacent slots.  Slices with a vtab row (filled before) are compared with it on
+// the way and marked as sharing it or not: 64^3 with equal coefficients, FP64, 299
+// us for the whole assembly (297 without the comparison; a pass of its own over the
+// stored values made it 353).
+template <typename VT, bool kShare>
 __global__ __launch_bounds__(kBlock) void k_sell_refresh(int64_t n, const uint32_t* __restrict__ sptr,
                                                          const int32_t* __restrict__ perm,
                                                          const int32_t* __restrict__ rowptr,
                                                          const uint32_t* __restrict__ kept,
                                                          const double* __restrict__ val64,
-                                                         VT* __restrict__ sval, int* flags) {
+                                                         VT* __restrict__ sval,
+                                                         const uint32_t* __restrict__ vptr,
+                                                         const SharedT<VT>* __restrict__ vtab,
+                                                         uint32_t* __restrict__ cptr, int* flags) {
   constexpr int G = 8, KT = 128;
   __shared__ double tile[kBlock / kSlice][G][KT + 1];
+  __shared__ SharedT<VT> vrow[kShare ? kBlock / kSlice : 1][kShare ? KT : 1];
   const int lane = threadIdx.x & (kSlice - 1);
   const int w = threadIdx.x >> 6;
   const int64_t s = (int64_t)blockIdx.x * (kBlock / kSlice) + w;
@@ -1720,15 +1718,25 @@ __global__ __launch_bounds__(kBlock) void k_sell_refresh(int64_t n, const uint32
   // lanes past the last row hold empty ranges, so every row index below 64
   // is safe
   int32_t b0 = 0, b1 = 0;
+  uint32_t vp = kShare ? vptr[s] : kNoShared;
   if (lane < rows) {
     const int64_t row = perm ? (int64_t)perm[t0 + lane] : t0 + lane;
     b0 = rowptr[row];
     b1 = rowptr[row + 1];
   }
+  // the vtab row that the slice's rows are compared with, if it has one: read once
+  // (a load per entry would lengthen every group's chain)
+  vp = (uint32_t)__builtin_amdgcn_readfirstlane((int)vp);
+  const bool shares = kShare && vp != kNoShared;
+  if (shares) {
+    const int last = (int)((sptr[s + 1] - sptr[s]) / kSlice) - 1;
+    vrow[w][lane] = vtab[vp + min(lane, last)];
+    vrow[w][lane + kSlice] = vtab[vp + min(lane + kSlice, last)];
+  }
   VT* base = sval + sptr[s];
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   double (*tl)[KT + 1] = tile[w];
-  bool bad = false;
+  bool bad = false, differs = false;
   for (int g0 = 0; g0 < rows; g0 += G) {
     int32_t len = 0;  // lane r < G: kept entries of row g0 + r
     for (int j0 = g0; j0 < g0 + G; j0 += 4) {
@@ -1757,7 +1765,11 @@ __global__ __launch_bounds__(kBlock) void k_sell_refresh(int64_t n, const uint32
           if (keep[u]) {
             const int32_t at = k[u] + __popcll(m & below);
             if (at < KT) tl[j0 - g0 + u][at] = v[u];
-            else base[j0 + u + (int64_t)at * kSlice] = (VT)v[u];
+            else {
+              const VT stored = (VT)v[u];
+              base[j0 + u + (int64_t)at * kSlice] = stored;
+              if (shares) differs |= !same_bits(ld(&stored), (double)vtab[vp + at]);
+            }
           } else if (in[u] && v[u] != 0.0) {
             bad = true;
           }
@@ -1777,11 +1789,66 @@ __global__ __launch_bounds__(kBlock) void k_sell_refresh(int64_t n, const uint32
     const int32_t mine = min(__shfl(len, r, 64), KT);
     for (int32_t kb = 0; kb < top; kb += kSlice / G) {
       const int32_t at = kb + (lane >> 3);
-      if (at < mine) base[g0 + r + (int64_t)at * kSlice] = (VT)tl[r][at];
+      const VT stored = (VT)tl[r][at];
+      if constexpr (kShare)
+        differs |= (int)(at < mine) & (int)!same_bits(ld(&stored), (double)vrow[w][at]);
+      if (at < mine) base[g0 + r + (int64_t)at * kSlice] = stored;
     }
     __builtin_amdgcn_wave_barrier();
   }
   if (bad) flags[1] = 1;
+  if (shares) {
+    const bool same = __ballot(differs) == 0;
+    if (lane == 0) cptr[s] = 0x60000000u | (same ? kSharedBit | vp : 0u);
+  }
+}
+
+// vsrc: the CSR entry behind each vtab entry, one wavefront per slice that stands
+// for a row: the kept entries of its first row, as k_sell_refresh stores them
+__global__ __launch_bounds__(kBlock) void k_vtab_src(int64_t nvrep, const int32_t* __restrict__ vrep,
+                                                     const uint32_t* __restrict__ vptr,
+                                                     const int32_t* __restrict__ perm,
+                                                     const int32_t* __restrict__ rowptr,
+                                                     const uint32_t* __restrict__ kept,
+                                                     int32_t* __restrict__ vsrc) {
+  const int64_t r = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
+  if (r >= nvrep) return;  // the whole wavefront
+  const int lane = threadIdx.x & (kSlice - 1);
+  const int64_t s = vrep[r];
+  const int64_t row = perm ? (int64_t)perm[s * kSlice] : s * kSlice;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  uint32_t at = vptr[s];
+  for (int32_t q0 = rowptr[row]; q0 < rowptr[row + 1]; q0 += kSlice) {
+    const int32_t q = q0 + lane;
+    const bool keep = q < rowptr[row + 1] && ((kept[q >> 5] >> (q & 31)) & 1u);
+    const uint64_t m = __ballot(keep);
+    if (keep) vsrc[at + __popcll(m & below)] = q;
+    at += __popcll(m);
+  }
+}
+
+// The inverse diagonals of a scalar matrix (workgroups up to ndiag, as
+// k_block_inverse<1>), and in the workgroups after them the vtab rows from the CSR
+// values.
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void k_diag_vtab(
+    int64_t n, unsigned ndiag, const int32_t* __restrict__ diagpos, const double* __restrict__ val64,
+    SharedT<VT>* __restrict__ dinv, int* __restrict__ singular, int64_t nvtab,
+    const int32_t* __restrict__ vsrc, SharedT<VT>* __restrict__ vtab) {
+  if (blockIdx.x < ndiag) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    double m[1] = {val64[diagpos[i]]};
+    if (gauss_jordan<1>(m))
+      dinv[i] = (SharedT<VT>)m[0];
+    else
+      atomicExch(singular, 1);
+    return;
+  }
+  const int64_t e = (int64_t)(blockIdx.x - ndiag) * kBlock + threadIdx.x;
+  if (e >= nvtab) return;
+  const VT stored = (VT)val64[vsrc[e]];
+  vtab[e] = (SharedT<VT>)ld(&stored);
 }
 
 int csr_asm_values(gh_ctx* ctx, gh_csr* A, double** val64) {
@@ -1825,42 +1892,45 @@ int csr_asm_commit(gh_ctx* ctx, gh_csr* A, const char* who) {
     GH_TRY(upload(ctx, &A->d_diag, diag.data(), n));
     GH_TRY(upload(ctx, &A->d_kept, kept.data(), (int64_t)kept.size()));
   }
-  // the assembly has written v64 on the stream; everything below follows it
-  if (A->prec == GH_F64)
-    GH_TRY(launch_block_inverse(ctx, n, 1, A->d_diag, v64, (double*)A->dinv, A->d_flags));
-  else
-    GH_TRY(launch_block_inverse(ctx, n, 1, A->d_diag, v64, (float*)A->dinv, A->d_flags));
-  if (A->prec == GH_F32)
-    hipLaunchKernelGGL((k_convert<float, double>), dim3(grid_stride(nnz)), dim3(kBlock), 0,
-                       ctx->stream, nnz, (float*)A->val, (const double*)v64);
-  else if (A->prec == GH_F16)
-    hipLaunchKernelGGL((k_convert<__half, double>), dim3(grid_stride(nnz)), dim3(kBlock), 0,
-                       ctx->stream, nnz, (__half*)A->val, (const double*)v64);
-  GH_HIP(hipGetLastError());
   const Sell& S = A->sell;
-  const int64_t nslices = (n + kSlice - 1) / kSlice;
-  const dim3 g((unsigned)std::max<int64_t>((nslices + kBlock / kSlice - 1) / (kBlock / kSlice), 1));
-  if (A->prec == GH_F64)
-    hipLaunchKernelGGL(k_sell_refresh<double>, g, dim3(kBlock), 0, ctx->stream, n, S.sptr, S.perm,
-                       A->rowptr, A->d_kept, v64, (double*)S.val, A->d_flags);
-  else if (A->prec == GH_F32)
-    hipLaunchKernelGGL(k_sell_refresh<float>, g, dim3(kBlock), 0, ctx->stream, n, S.sptr, S.perm,
-                       A->rowptr, A->d_kept, v64, (float*)S.val, A->d_flags);
-  else
-    hipLaunchKernelGGL(k_sell_refresh<__half>, g, dim3(kBlock), 0, ctx->stream, n, S.sptr, S.perm,
-                       A->rowptr, A->d_kept, v64, (__half*)S.val, A->d_flags);
-  GH_HIP(hipGetLastError());
-  // which slices share values now; flag [3] counts their entries
-  if (S.vtab) {
-    hipLaunchKernelGGL(k_fill0<int>, dim3(1), dim3(kBlock), 0, ctx->stream, (int64_t)1,
-                       A->d_flags + 3);
-    GH_TRY(sell_share(ctx, S, A->d_flags + 3));
+  if (S.vtab && !S.vsrc) {
+    if (hipMalloc((void**)&A->sell.vsrc, sizeof(int32_t) * S.nvtab) != hipSuccess)
+      return fail(GH_ENOMEM, "%s: shared values", who);
+    hipLaunchKernelGGL(k_vtab_src, dim3(grid_for(S.nvrep, kBlock / kSlice)), dim3(kBlock), 0,
+                       ctx->stream, S.nvrep, S.vrep, S.vptr, S.perm, A->rowptr, A->d_kept, S.vsrc);
+    GH_HIP(hipGetLastError());
   }
+  // the assembly has written v64 on the stream; everything below follows it
+  auto commit = [&](auto vt) -> int {
+    using VT = decltype(vt);
+    if (S.vtab) {
+      const unsigned nd = grid_for(n);
+      hipLaunchKernelGGL(k_diag_vtab<VT>, dim3(nd + grid_for(S.nvtab)), dim3(kBlock), 0, ctx->stream,
+                         n, nd, A->d_diag, v64, (SharedT<VT>*)A->dinv, A->d_flags, S.nvtab, S.vsrc,
+                         (SharedT<VT>*)S.vtab);
+    } else {
+      GH_TRY(launch_block_inverse(ctx, n, 1, A->d_diag, v64, (SharedT<VT>*)A->dinv, A->d_flags));
+    }
+    if constexpr (!std::is_same<VT, double>::value)
+      hipLaunchKernelGGL((k_convert<VT, double>), dim3(grid_stride(nnz)), dim3(kBlock), 0, ctx->stream,
+                         nnz, (VT*)A->val, (const double*)v64);
+    const auto refresh = S.vtab ? k_sell_refresh<VT, true> : k_sell_refresh<VT, false>;
+    hipLaunchKernelGGL(refresh, dim3(grid_for(S.nslices, kBlock / kSlice)), dim3(kBlock), 0,
+                       ctx->stream, n, S.sptr, S.perm, A->rowptr, A->d_kept, v64, (VT*)S.val, S.vptr,
+                       (const SharedT<VT>*)S.vtab, S.cptr, A->d_flags);
+    GH_HIP(hipGetLastError());
+    return GH_OK;
+  };
+  if (A->prec == GH_F64)
+    GH_TRY(commit(double{}));
+  else if (A->prec == GH_F32)
+    GH_TRY(commit(float{}));
+  else
+    GH_TRY(commit(__half{}));
   int flags[4] = {0, 0, 0, 0};
   GH_HIP(hipMemcpyAsync(flags, A->d_flags, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
   GH_HIP(hipStreamSynchronize(ctx->stream));
   A->h_val_ok = false;
-  A->sell.shared = S.vtab ? (uint32_t)flags[3] : 0;
   if (flags[0] || flags[1] || flags[2]) {
     GH_HIP(hipMemsetAsync(A->d_flags, 0, sizeof(int) * 4, ctx->stream));
     GH_HIP(hipStreamSynchronize(ctx->stream));
@@ -2086,7 +2156,23 @@ int gh_csr_layout(const gh_csr* A, int64_t* out) {
   return GH_OK;
 }
 
-int64_t gh_csr_shared_entries(const gh_csr* A) { return A ? A->sell.shared : 0; }
+int64_t gh_csr_shared_entries(const gh_csr* A) {
+  if (!A || !A->sell.vtab) return 0;
+  const Sell& S = A->sell;
+  std::vector<uint32_t> cptr(S.nslices), sptr(S.nslices + 1);
+  if (hipMemcpyAsync(cptr.data(), S.cptr, 4 * cptr.size(), hipMemcpyDeviceToHost, A->ctx->stream) !=
+          hipSuccess ||
+      hipMemcpyAsync(sptr.data(), S.sptr, 4 * sptr.size(), hipMemcpyDeviceToHost, A->ctx->stream) !=
+          hipSuccess ||
+      hipStreamSynchronize(A->ctx->stream) != hipSuccess)
+    return fail(GH_EHIP, "gh_csr_shared_entries: download failed");
+  constexpr uint32_t kShares = 0x60000000u | kSharedBit;
+  int64_t entries = 0;
+  for (int64_t s = 0; s < S.nslices; ++s)
+    if ((cptr[s] & kShares) == kShares && !(cptr[s] & 0x80000000u))
+      entries += std::min<int64_t>(kSlice, S.n - s * kSlice) * ((sptr[s + 1] - sptr[s]) / kSlice);
+  return entries;
+}
 
 int gh_csr_waves(const gh_csr* A) {
   if (!A || A->host_only) return 0;

@@ -139,15 +139,15 @@ struct Sell {
   int64_t npat = 0, ntab = 0;
   // shared values (slices of one pattern whose 64 rows also hold the same values,
   // entry by entry, as stored): cptr bit 28 and, in bits 0..27, the place of that
-  // row in vtab (double for FP64 storage, else float).  vptr / vrep: per slice
-  // the place its row would take (0xFFFFFFFF: none) and the slice it is taken
-  // from; whether a slice shares is found again whenever the values change
-  // (sell_share).
+  // row in vtab (double for FP64 storage, else float).  vptr: per slice the place
+  // of its row (0xFFFFFFFF: none); vrep: the slices whose first rows fill vtab;
+  // vsrc: the CSR entry behind each vtab entry (made by the first assembly).
+  // Whether a slice shares is found again whenever the values change.
   void* vtab = nullptr;
   uint32_t* vptr = nullptr;
   int32_t* vrep = nullptr;
-  int64_t nvtab = 0;
-  int64_t shared = 0;        // stored entries whose values come from vtab
+  int32_t* vsrc = nullptr;
+  int64_t nvrep = 0, nvtab = 0;
   int64_t patterned = 0;     // slices in pattern mode
   int64_t single = 0;        // slots of the slices whose rows share one pattern
   int64_t col_bytes = 0;     // column bytes a sweep reads (stored entries only)
@@ -194,9 +194,6 @@ void bsell_free(BSell* S);
 int sell_build(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const uint32_t* col,
                const double* vals, int prec, Sell* S);
 void sell_free(Sell* S);
-// Fill vtab from the slices' present values and mark the slices that share;
-// count (device, zero before) += their stored entries.
-int sell_share(gh_ctx* ctx, const Sell& S, int* count);
 
 }  // namespace gh
 
@@ -263,8 +260,7 @@ struct gh_csr {
   uint32_t* d_kept = nullptr;  // bit q: CSR entry q is stored in the SELL layout
   double* d_val64 = nullptr;   // FP64 CSR values of a reduced-precision matrix
   int* d_flags = nullptr;      // [0] singular diagonal, [1] a left-out entry became nonzero,
-                               // [2] an element coupling has no entry in the pattern,
-                               // [3] entries of slices that share values
+                               // [2] an element coupling has no entry in the pattern
   int asm_mode = -1;           // how the Q2 device assembly finds entries (found on first use)
   int cols_ascend = -1;        // 1: every row's columns ascend (found on first use)
 };

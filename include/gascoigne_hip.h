@@ -135,7 +135,8 @@ int gh_csr_prec(const gh_csr* A);
  * out[2..5] = 0, out[6] = 4 nnz, out[7] = 0. */
 int gh_csr_layout(const gh_csr* A, int64_t* out);
 /* stored entries whose values a sweep takes from rows shared by whole slices
- * (a slice whose 64 rows hold equal values stores them, but does not read them) */
+ * (a slice whose 64 rows hold equal values stores them, but does not read them);
+ * negative: an error.  Synchronises. */
 int64_t gh_csr_shared_entries(const gh_csr* A);
 /* wavefronts that share a slice of 64 rows in products of FP64 vectors: 1, 4
  * or 8 (the results are the same, bit for bit); 0 without a device layout */
