@@ -635,40 +635,6 @@ constexpr int kMaxSlicePatterns = 16;
 
 // orig: original row of each slot (nullptr: slot = row); rowptr/col/vals are
 // already in slot order.
-// A table from 64-bit keys (the row-pattern hashes) to counters or row
-// indices: open addressing with linear probing, sized for n keys; it stands
-// in for std::unordered_map where millions of rows are looked up.
-struct KeyTable {
-  std::vector<uint64_t> key;
-  std::vector<int64_t> val;
-  std::vector<uint8_t> used;
-  uint64_t mask = 0;
-  KeyTable(int64_t n, int64_t init) {
-    uint64_t cap = 16;
-    while (cap < 2 * (uint64_t)std::max<int64_t>(n, 1)) cap <<= 1;
-    key.assign(cap, 0);
-    val.assign(cap, init);
-    used.assign(cap, 0);
-    mask = cap - 1;
-    fill = init;
-  }
-  // the value of k, inserted with the initial value if absent
-  int64_t& operator[](uint64_t k) {
-    uint64_t h = (k * 0x9E3779B97F4A7C15ull) >> 17;
-    for (;; ++h) {
-      const uint64_t b = h & mask;
-      if (!used[b]) {
-        used[b] = 1;
-        key[b] = k;
-        val[b] = fill;
-        return val[b];
-      }
-      if (key[b] == k) return val[b];
-    }
-  }
-  int64_t fill = 0;
-};
-
 // ------------------------------------------------------------ shared values
 constexpr uint32_t kNoShared = 0xFFFFFFFFu;  // vptr of a slice without a vtab row
 
@@ -756,17 +722,18 @@ __global__ __launch_bounds__(kBlock) void k_sell_mark(int64_t n, int64_t nslices
 
 // Finds the slices that share values when the layout is built: slices of one
 // pattern with equal value hashes take one vtab row.
-static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& one) {
+static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& one,
+                            const std::vector<uint32_t>& cb, const std::vector<int32_t>& ps) {
   const int64_t ns = S->nslices;
   bool any = false;
   for (int64_t s = 0; s < ns && !any; ++s) any = one[s] != 0;
   if (!any) return GH_OK;
+  // the hashes, then vptr and vrep in their place
   uint64_t* d_hash = nullptr;
   if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * ns) != hipSuccess)
     return fail(GH_ENOMEM, "sell_build: allocation failed");
   std::vector<uint64_t> hash(ns);
-  std::vector<uint32_t> cb(ns), vptr(ns, kNoShared);
-  std::vector<int32_t> vrep, ps(S->npat + 1);
+  std::vector<uint32_t> lists(ns, kNoShared);
   auto run = [&]() -> int {
     const dim3 g(grid_for(ns, kBlock / kSlice)), b(kBlock);
     if (S->prec == GH_F64)
@@ -780,34 +747,33 @@ static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& on
                          S->cbase, S->pstart, (const __half*)S->val, d_hash);
     GH_HIP(hipGetLastError());
     GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
-    GH_HIP(hipMemcpyAsync(cb.data(), S->cbase, sizeof(uint32_t) * ns, hipMemcpyDeviceToHost, ctx->stream));
-    GH_HIP(hipMemcpyAsync(ps.data(), S->pstart, sizeof(int32_t) * ps.size(), hipMemcpyDeviceToHost,
-                          ctx->stream));
     GH_HIP(hipStreamSynchronize(ctx->stream));
-    std::unordered_map<uint64_t, int32_t> first;
+    KeyTable first(ns, -1);
     int64_t total = 0;
     for (int64_t s = 0; s < ns; ++s) {
       if (!hash[s]) continue;
       const int32_t len = ps[cb[s] + 1] - ps[cb[s]];
-      auto it = first.emplace(hash[s], (int32_t)s).first;
-      const int64_t r = it->second;
+      int64_t& r = first[hash[s]];
+      if (r < 0) r = s;
       if (r != s && cb[r] != cb[s]) continue;  // equal hashes of two patterns
       if (r == s) {
         if (total + len > (int64_t)kSharedMask) continue;
-        vptr[s] = (uint32_t)total;
+        lists[s] = (uint32_t)total;
         total += len;
-        vrep.push_back((int32_t)s);
+        lists.push_back((uint32_t)s);
       } else {
-        vptr[s] = vptr[r];
+        lists[s] = lists[r];
       }
     }
     if (total == 0) return GH_OK;
-    S->nvrep = (int64_t)vrep.size();
+    S->nvrep = (int64_t)lists.size() - ns;
     S->nvtab = total;
     if (hipMalloc(&S->vtab, total * (S->prec == GH_F64 ? 8 : 4)) != hipSuccess)
       return fail(GH_ENOMEM, "sell_build: allocation failed");
-    GH_TRY(upload(ctx, &S->vptr, vptr.data(), vptr.size()));
-    GH_TRY(upload(ctx, &S->vrep, vrep.data(), vrep.size()));
+    S->vptr = (uint32_t*)d_hash;
+    S->vrep = (int32_t*)(S->vptr + ns);
+    GH_HIP(hipMemcpyAsync(S->vptr, lists.data(), sizeof(uint32_t) * lists.size(), hipMemcpyHostToDevice,
+                          ctx->stream));
     auto mark = [&](auto vt) -> int {
       using VT = decltype(vt);
       hipLaunchKernelGGL(k_sell_vtab<VT>, dim3(grid_for(S->nvrep, kBlock / kSlice)), b, 0, ctx->stream,
@@ -824,7 +790,7 @@ static int sell_share_build(gh_ctx* ctx, Sell* S, const std::vector<uint8_t>& on
     return mark(__half{});
   };
   const int rc = run();
-  (void)hipFree(d_hash);
+  if (!S->vptr) (void)hipFree(d_hash);
   return rc;
 }
 
@@ -1122,7 +1088,7 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
     (void)hipFree(tmp);
   }
   GH_HIP(hipStreamSynchronize(ctx->stream));
-  return sell_share_build(ctx, S, one);
+  return sell_share_build(ctx, S, one, cbase, pstart);
 }
 
 // Valued operators: the rows of a window of kSellWindow rows may run in
@@ -1260,7 +1226,7 @@ int sell_build(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const uint32_t* co
 void sell_free(Sell* S) {
   for (void* p : {(void*)S->sptr, (void*)S->rlen, (void*)S->col, S->val, (void*)S->cidx,
                   (void*)S->cptr, (void*)S->cbase, (void*)S->ptab, (void*)S->pstart,
-                  (void*)S->perm, S->vtab, (void*)S->vptr, (void*)S->vrep, (void*)S->vsrc})
+                  (void*)S->perm, S->vtab, (void*)S->vptr, (void*)S->vsrc})
     if (p) (void)hipFree(p);
   S->vtab = nullptr;
   S->vptr = nullptr;

@@ -27,14 +27,15 @@ struct gh_vanka {
   int64_t nclasses = 0;       // distinct patch matrices
   int ld = 0;                 // entries of a factor column: m rounded up to 16, zeros below row m
   int64_t lstride = 0;        // entries of one class's factors: ld * m
+  int32_t* ints = nullptr;    // all lists below
   int32_t* nodes = nullptr;   // npatches * psize
   int32_t* cls = nullptr;     // class of each patch
   void* lu = nullptr;         // nclasses * lstride, column-major, L unit lower
-  double* rdiag = nullptr;    // nclasses * m: 1 / u_kk, 0 where it is not used
+  double* rdiag = nullptr;    // nclasses * m, behind lu: 1 / u_kk, 0 where it is not used
   int32_t* piv = nullptr;     // npatches * m: the global entry gathered into each factor row
   int32_t* nptr = nullptr;    // n + 1
   int32_t* nent = nullptr;    // patch * psize + local node, ascending patch per node
-  void* xp = nullptr;         // npatches * m local solutions
+  void* xp = nullptr;         // npatches * m local solutions (scratch at creation)
   // grouped solve: workgroup g takes the patches plist[first .. first + count)
   // of one class; (class, first, count) per group.  ngroups = 0: one wavefront
   // per patch instead
@@ -109,6 +110,40 @@ inline unsigned grid_for(int64_t work, int per_block = kBlock) {
   return (unsigned)g;
 }
 
+// A table from 64-bit keys (hashes of row patterns or patch matrices) to counters or
+// indices: open addressing with linear probing, sized for n keys; it stands
+// in for std::unordered_map where millions of rows are looked up.
+struct KeyTable {
+  std::vector<uint64_t> key;
+  std::vector<int64_t> val;
+  std::vector<uint8_t> used;
+  uint64_t mask = 0;
+  KeyTable(int64_t n, int64_t init) {
+    uint64_t cap = 16;
+    while (cap < 2 * (uint64_t)std::max<int64_t>(n, 1)) cap <<= 1;
+    key.assign(cap, 0);
+    val.assign(cap, init);
+    used.assign(cap, 0);
+    mask = cap - 1;
+    fill = init;
+  }
+  // the value of k, inserted with the initial value if absent
+  int64_t& operator[](uint64_t k) {
+    uint64_t h = (k * 0x9E3779B97F4A7C15ull) >> 17;
+    for (;; ++h) {
+      const uint64_t b = h & mask;
+      if (!used[b]) {
+        used[b] = 1;
+        key[b] = k;
+        val[b] = fill;
+        return val[b];
+      }
+      if (key[b] == k) return val[b];
+    }
+  }
+  int64_t fill = 0;
+};
+
 // number of device scalar slots for reduction results
 constexpr int kScalars = 512;
 
@@ -145,7 +180,7 @@ struct Sell {
   // Whether a slice shares is found again whenever the values change.
   void* vtab = nullptr;
   uint32_t* vptr = nullptr;
-  int32_t* vrep = nullptr;
+  int32_t* vrep = nullptr;   // behind vptr
   int32_t* vsrc = nullptr;
   int64_t nvrep = 0, nvtab = 0;
   int64_t patterned = 0;     // slices in pattern mode

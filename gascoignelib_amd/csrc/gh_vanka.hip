@@ -130,26 +130,45 @@ __device__ __forceinline__ void factor_columns(int m, int tr, int tc,
   }
 }
 
+// A patch's nodes and their places, open addressing (at most half full).
+struct PatchMap {
+  static constexpr int kSize = 2 * kVankaMaxNodes;
+  int32_t node[kSize], place[kSize];
+  static __device__ __forceinline__ int hash(int32_t v) {
+    return (int)(((uint32_t)v * 0x9E3779B1u) >> 24);
+  }
+};
+static_assert(PatchMap::kSize == 256, "hash: 8 bits");
+
 // copy_entries_sparseblockmatrix: tab[r * psize + u] = CSR position of the block
 // (patch node r, patch node u), -1 where the matrix has none.  All NT threads of
-// the workgroup; NT / psize of them walk each row's entries.  Ends in a barrier.
+// the workgroup; NT / psize of them walk each row's entries and look the columns
+// up.  Ends in a barrier.
 template <int NT>
 __device__ __forceinline__ void patch_positions(int psize, const int32_t* __restrict__ nodes,
                                                 const int32_t* __restrict__ rowptr,
                                                 const int32_t* __restrict__ col, int32_t* tab,
-                                                int32_t* pn) {
+                                                PatchMap& map) {
+  constexpr int last = PatchMap::kSize - 1;
   const int t = threadIdx.x;
   for (int e = t; e < psize * psize; e += NT) tab[e] = -1;
-  for (int r = t; r < psize; r += NT) pn[r] = nodes[r];
+  for (int e = t; e <= last; e += NT) map.node[e] = -1;
+  __syncthreads();
+  for (int r = t; r < psize; r += NT) {  // distinct nodes: each takes a free slot
+    int h = PatchMap::hash(nodes[r]);
+    while (atomicCAS(&map.node[h], -1, nodes[r]) != -1) h = (h + 1) & last;
+    map.place[h] = r;
+  }
   __syncthreads();
   const int per = NT / psize;
   const int r = t / per, u0 = t - r * per;
   if (r < psize) {
-    const int32_t row = pn[r];
+    const int32_t row = nodes[r];
     for (int32_t q = rowptr[row] + u0; q < rowptr[row + 1]; q += per) {
       const int32_t c0 = col[q];
-      for (int u = 0; u < psize; ++u)
-        if (pn[u] == c0) tab[r * psize + u] = q;
+      int h = PatchMap::hash(c0);
+      while (map.node[h] != c0 && map.node[h] != -1) h = (h + 1) & last;
+      if (map.node[h] == c0) tab[r * psize + map.place[h]] = q;
     }
   }
   __syncthreads();
@@ -162,7 +181,7 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-constexpr int kHashThreads = 256;
+constexpr int kHashThreads = 1024;  // as many walk a row: 64 patches of 108, creation 0.34 ms with 256
 
 // Two 64-bit sums over the patch matrix's entries, each entry's bits mixed with
 // its place: equal matrices have equal sums, and the patches with equal sums are
@@ -171,11 +190,11 @@ __global__ __launch_bounds__(kHashThreads) void k_vanka_hash(
     int psize, int B, const int32_t* __restrict__ nodes, const int32_t* __restrict__ rowptr,
     const int32_t* __restrict__ col, const double* __restrict__ val, uint64_t* __restrict__ out) {
   extern __shared__ int32_t tab[];
-  __shared__ int32_t pn[kVankaMaxNodes];
+  __shared__ PatchMap map;
   __shared__ uint64_t part[2][kHashThreads / 64];
   const int64_t p = blockIdx.x;
   const int BB = B * B, t = threadIdx.x;
-  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, pn);
+  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, map);
   uint64_t h0 = 0, h1 = 0;
   for (int e = t; e < psize * psize * BB; e += kHashThreads) {
     const int32_t q = tab[e / BB];
@@ -200,24 +219,30 @@ __global__ __launch_bounds__(kHashThreads) void k_vanka_hash(
   }
 }
 
-// flag[p] = 1 where patch p's matrix differs from patch rep[p]'s in any bit
+// flag[p]: whether patch p's matrix differs from patch rep[p]'s in any bit
 __global__ __launch_bounds__(kHashThreads) void k_vanka_same(
     int psize, int B, const int32_t* __restrict__ nodes, const int32_t* __restrict__ rowptr,
     const int32_t* __restrict__ col, const double* __restrict__ val,
     const int32_t* __restrict__ rep, int32_t* __restrict__ flag) {
   extern __shared__ int32_t tab[];  // 2 * psize * psize
-  __shared__ int32_t pn[kVankaMaxNodes];
+  __shared__ PatchMap map;
   const int64_t p = blockIdx.x, r = rep[p];
-  if (r == p) return;  // the whole workgroup
+  if (r == p) {  // the whole workgroup
+    if (threadIdx.x == 0) flag[p] = 0;
+    return;
+  }
   const int BB = B * B, PP = psize * psize;
-  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, pn);
-  patch_positions<kHashThreads>(psize, nodes + r * psize, rowptr, col, tab + PP, pn);
+  patch_positions<kHashThreads>(psize, nodes + p * psize, rowptr, col, tab, map);
+  patch_positions<kHashThreads>(psize, nodes + r * psize, rowptr, col, tab + PP, map);
+  int differs = 0;
   for (int e = threadIdx.x; e < PP * BB; e += kHashThreads) {
     const int32_t q = tab[e / BB], s = tab[PP + e / BB];
     const double x = q >= 0 ? val[(int64_t)q * BB + e % BB] : 0.0;
     const double y = s >= 0 ? val[(int64_t)s * BB + e % BB] : 0.0;
-    if (__builtin_bit_cast(uint64_t, x) != __builtin_bit_cast(uint64_t, y)) flag[p] = 1;
+    differs |= __builtin_bit_cast(uint64_t, x) != __builtin_bit_cast(uint64_t, y);
   }
+  differs = __syncthreads_or(differs);
+  if (threadIdx.x == 0) flag[p] = differs;
 }
 
 // LU with partial pivoting of every class's patch matrix, the oracle's operations in
@@ -231,12 +256,12 @@ __global__ __launch_bounds__(kFactorThreads, 8) void k_vanka_factor(
     const double* __restrict__ val, int ld, double* __restrict__ lu64,
     float* __restrict__ lu32, int32_t* __restrict__ piv) {
   extern __shared__ int32_t tab[];  // psize * psize CSR positions of the node blocks, -1: none
-  __shared__ int32_t pn[kVankaMaxNodes];
+  __shared__ PatchMap map;
   __shared__ FactorShared S;
   const int64_t p = blockIdx.x;
   const int m = psize * B;
   const int t = threadIdx.x, tr = t % kFactorLanes, tc = t / kFactorLanes;
-  patch_positions<kFactorThreads>(psize, nodes + (int64_t)reps[p] * psize, rowptr, col, tab, pn);
+  patch_positions<kFactorThreads>(psize, nodes + (int64_t)reps[p] * psize, rowptr, col, tab, map);
   double a[kRowsPer][kColsPer];
   int pos[kRowsPer];  // position of row tr + 64 i in the exchanged order; -1: no row
 #pragma unroll
@@ -266,6 +291,11 @@ __global__ __launch_bounds__(kFactorThreads, 8) void k_vanka_factor(
   // column-major factors (coalesced column reads in the solve), rows in the
   // exchanged order
   const int64_t base = p * (int64_t)ld * m;
+  for (int e = t; e < (ld - m) * m; e += kFactorThreads) {  // zeros below row m
+    const int64_t z = base + (int64_t)(e / (ld - m)) * ld + m + e % (ld - m);
+    if (lu64) lu64[z] = 0.0;
+    else lu32[z] = 0.0f;
+  }
 #pragma unroll
   for (int i = 0; i < kRowsPer; ++i) {
     if (pos[i] < 0) continue;
@@ -766,80 +796,46 @@ int vanka_apply_t(gh_ctx* ctx, const gh_vanka* V, const T* in, T* out, int mode,
   return GH_OK;
 }
 
-// The patches by class: cls[p], and reps[c] the first patch of class c (classes
-// in order of first appearance).  Patches whose hashes agree but whose entries
-// do not each get a class of their own.
-int patch_classes(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, int B,
-                  const int32_t* d_nodes, std::vector<int32_t>& cls, std::vector<int32_t>& reps) {
+// The first patch with each patch's matrix, by hash (`first`; the entries are
+// compared afterwards, k_vanka_same).  scratch: 2 * npatches 64-bit words.
+int patch_firsts(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, int B,
+                 const int32_t* d_nodes, void* scratch, std::vector<int32_t>& first) {
   const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
-  uint64_t* d_hash = nullptr;
-  int32_t* d_rep = nullptr;
+  uint64_t* d_hash = (uint64_t*)scratch;
   std::vector<uint64_t> hash(2 * npatches);
-  std::vector<int32_t> first(npatches), differs(npatches, 0);
-  int rc = GH_OK;
-  auto run = [&]() -> int {
-    if (hipMalloc((void**)&d_hash, sizeof(uint64_t) * 2 * npatches) != hipSuccess ||
-        hipMalloc((void**)&d_rep, sizeof(int32_t) * 2 * npatches) != hipSuccess)
-      return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
-    GH_HIP(hipFuncSetAttribute((const void*)k_vanka_hash,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    GH_HIP(hipFuncSetAttribute((const void*)k_vanka_same,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * lds)));
-    hipLaunchKernelGGL(k_vanka_hash, dim3((unsigned)npatches), dim3(kHashThreads), lds,
-                       ctx->stream, psize, B, d_nodes, A->rowptr, A->col, (const double*)A->val,
-                       d_hash);
-    GH_HIP(hipGetLastError());
-    GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * hash.size(),
-                          hipMemcpyDeviceToHost, ctx->stream));
-    GH_HIP(hipStreamSynchronize(ctx->stream));
-    bool shared = false;
-    {
-      // both sums must agree; the first patch with a pair stands for it
-      std::vector<int32_t> by(npatches);
-      for (int64_t p = 0; p < npatches; ++p) by[p] = (int32_t)p;
-      std::sort(by.begin(), by.end(), [&](int32_t a, int32_t b) {
-        if (hash[2 * a] != hash[2 * b]) return hash[2 * a] < hash[2 * b];
-        if (hash[2 * a + 1] != hash[2 * b + 1]) return hash[2 * a + 1] < hash[2 * b + 1];
-        return a < b;
-      });
-      int32_t f = npatches > 0 ? by[0] : 0;
-      for (int64_t i = 0; i < npatches; ++i) {
-        const int32_t p = by[i];
-        if (hash[2 * p] != hash[2 * f] || hash[2 * p + 1] != hash[2 * f + 1]) f = p;
-        first[p] = f;
-        shared = shared || f != p;
-      }
-    }
-    if (shared) {
-      GH_HIP(hipMemcpyAsync(d_rep, first.data(), sizeof(int32_t) * npatches, hipMemcpyHostToDevice,
-                            ctx->stream));
-      GH_HIP(hipMemcpyAsync(d_rep + npatches, differs.data(), sizeof(int32_t) * npatches,
-                            hipMemcpyHostToDevice, ctx->stream));
-      hipLaunchKernelGGL(k_vanka_same, dim3((unsigned)npatches), dim3(kHashThreads), 2 * lds,
-                         ctx->stream, psize, B, d_nodes, A->rowptr, A->col,
-                         (const double*)A->val, d_rep, d_rep + npatches);
-      GH_HIP(hipGetLastError());
-      GH_HIP(hipMemcpyAsync(differs.data(), d_rep + npatches, sizeof(int32_t) * npatches,
-                            hipMemcpyDeviceToHost, ctx->stream));
-      GH_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    return GH_OK;
-  };
-  rc = run();
-  if (d_hash) (void)hipFree(d_hash);
-  if (d_rep) (void)hipFree(d_rep);
-  GH_TRY(rc);
-  cls.assign(npatches, -1);
+  GH_HIP(hipFuncSetAttribute((const void*)k_vanka_hash,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(k_vanka_hash, dim3((unsigned)npatches), dim3(kHashThreads), lds, ctx->stream,
+                     psize, B, d_nodes, A->rowptr, A->col, (const double*)A->val, d_hash);
+  GH_HIP(hipGetLastError());
+  GH_HIP(hipMemcpyAsync(hash.data(), d_hash, sizeof(uint64_t) * hash.size(), hipMemcpyDeviceToHost,
+                        ctx->stream));
+  GH_HIP(hipStreamSynchronize(ctx->stream));
+  KeyTable table(npatches, -1);
+  first.resize(npatches);
+  for (int64_t p = 0; p < npatches; ++p) {
+    int64_t& f = table[hash[2 * p] ^ (hash[2 * p + 1] * 0x9E3779B97F4A7C15ull)];
+    if (f < 0) f = p;
+    first[p] = (int32_t)f;
+  }
+  return GH_OK;
+}
+
+// The patches by class: cls[p], and reps[c] the first patch of class c (classes
+// in order of first appearance).  A patch that differs from its first has a class
+// of its own.
+void patch_classes(const std::vector<int32_t>& first, const std::vector<int32_t>& differs,
+                   std::vector<int32_t>& cls, std::vector<int32_t>& reps) {
+  cls.assign(first.size(), -1);
   reps.clear();
-  for (int64_t p = 0; p < npatches; ++p) {  // first[p] <= p
-    if (first[p] == p || differs[p]) {
+  for (size_t p = 0; p < first.size(); ++p) {  // first[p] <= p
+    if (first[p] == (int32_t)p || differs[p]) {
       cls[p] = (int32_t)reps.size();
       reps.push_back((int32_t)p);
     } else {
       cls[p] = cls[first[p]];
     }
   }
-  return GH_OK;
 }
 
 // Whether the grouped solve runs, and its groups: chunks of a class's patches, as
@@ -861,10 +857,11 @@ int patch_classes(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, int
 // 25 us against 40, 44, 38, 44 and 38; 81 unknowns (two per CU), 8192 patches in
 // classes of 2, 3, 4: 139, 103, 76 against 106, 102, 100; 54 unknowns, classes of 2:
 // 54 against 59.
-int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
+void vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls,
+                  std::vector<int32_t>& plist, std::vector<int32_t>& groups) {
   const int64_t np = V->npatches, nc = V->nclasses;
   const int64_t fit = V->prec == GH_F64 ? group_fit<double>(V->m) : group_fit<float>(V->m);
-  if (fit < 1) return GH_OK;
+  if (fit < 1) return;
   const int64_t at_once = fit * ctx->num_cu;
   std::vector<int64_t> start(nc + 1, 0);
   for (int64_t p = 0; p < np; ++p) start[cls[p] + 1]++;
@@ -885,9 +882,9 @@ int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
     const int64_t rounds = (nc + at_once - 1) / at_once;
     if (c >= most || (g <= at_once && np >= least * g) || rounds * (2 + c / kPass) > best) break;
   }
-  if (np < least * ng || (ng > at_once && np * fit < (least + 2) * ng)) return GH_OK;
+  if (np < least * ng || (ng > at_once && np * fit < (least + 2) * ng)) return;
   for (int64_t c = 0; c < nc; ++c) start[c + 1] += start[c];
-  std::vector<int32_t> plist(np), groups;
+  plist.resize(np);
   {
     std::vector<int64_t> fill(start.begin(), start.end() - 1);
     for (int64_t p = 0; p < np; ++p) plist[fill[cls[p]]++] = (int32_t)p;
@@ -898,13 +895,7 @@ int vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls) {
       groups.push_back((int32_t)a);
       groups.push_back((int32_t)std::min(chunk, start[c + 1] - a));
     }
-  if (hipMalloc((void**)&V->plist, sizeof(int32_t) * np) != hipSuccess ||
-      hipMalloc((void**)&V->groups, sizeof(int32_t) * groups.size()) != hipSuccess)
-    return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
-  GH_HIP(hipMemcpy(V->plist, plist.data(), sizeof(int32_t) * np, hipMemcpyHostToDevice));
-  GH_HIP(hipMemcpy(V->groups, groups.data(), sizeof(int32_t) * groups.size(), hipMemcpyHostToDevice));
   V->ngroups = (int64_t)groups.size() / 3;
-  return GH_OK;
 }
 
 }  // namespace
@@ -964,39 +955,52 @@ int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, cons
     gh_vanka_destroy(V);
     return rc;
   };
+  // Few allocations and copies, since they are most of what the creation of a small
+  // level costs (64 patches of 108: 0.26 ms).  ints: nodes, nptr, nent; then per
+  // factorisation cls, reps; then the gather, plist and groups.
   const size_t ts = prec == GH_F64 ? 8 : 4;
-  auto alloc = [&](void** p, size_t bytes) {
-    return hipMalloc(p, std::max<size_t>(bytes, 8)) == hipSuccess;
-  };
-  if (!alloc((void**)&V->nodes, sizeof(int32_t) * npatches * psize) ||
-      !alloc((void**)&V->cls, sizeof(int32_t) * npatches) ||
-      !alloc((void**)&V->piv, sizeof(int32_t) * npatches * m) ||
-      !alloc((void**)&V->nptr, sizeof(int32_t) * (n + 1)) ||
-      !alloc((void**)&V->nent, sizeof(int32_t) * npatches * psize) ||
-      !alloc(&V->xp, ts * npatches * m))
+  const int64_t np = npatches, ne = np * psize;
+  if (hipMalloc((void**)&V->ints, sizeof(int32_t) * (2 * ne + (n + 1) + np * (m + 6))) != hipSuccess ||
+      hipMalloc(&V->xp, std::max<size_t>({ts * np * m, sizeof(int32_t) * np * (m + 2),
+                                          sizeof(uint64_t) * 2 * np, 8})) != hipSuccess)
     return bail(fail(GH_ENOMEM, "gh_vanka_create: allocation failed"));
-  if (hipMemcpy(V->nodes, nodes, sizeof(int32_t) * npatches * psize, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(V->nptr, nptr.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(V->nent, nent.data(), sizeof(int32_t) * npatches * psize, hipMemcpyHostToDevice) != hipSuccess)
-    return bail(fail(GH_EHIP, "gh_vanka_create: upload failed"));
+  V->nodes = V->ints;
+  V->nptr = V->nodes + ne;
+  V->nent = V->nptr + n + 1;
+  V->cls = V->nent + ne;
+  int32_t* d_reps = V->cls + np;
+  V->piv = d_reps + np;
+  V->plist = V->piv + np * m;
+  V->groups = V->plist + np;  // at most one per patch
+  {
+    std::vector<int32_t> up(2 * ne + n + 1);
+    std::copy(nodes, nodes + ne, up.begin());
+    std::copy(nptr.begin(), nptr.end(), up.begin() + ne);
+    std::copy(nent.begin(), nent.end(), up.begin() + ne + n + 1);
+    if (hipMemcpy(V->nodes, up.data(), sizeof(int32_t) * up.size(), hipMemcpyHostToDevice) != hipSuccess)
+      return bail(fail(GH_EHIP, "gh_vanka_create: upload failed"));
+  }
   if (npatches > 0) {
-    std::vector<int32_t> cls, reps;
-    if (int rc = patch_classes(ctx, A, npatches, psize, B, V->nodes, cls, reps)) return bail(rc);
-    const int64_t nc = V->nclasses = (int64_t)reps.size();
+    std::vector<int32_t> first, cls, reps, piv, differs(np, 0);
+    if (int rc = patch_firsts(ctx, A, np, psize, B, V->nodes, V->xp, first)) return bail(rc);
     V->ld = (m + 15) / 16 * 16;
     V->lstride = (int64_t)V->ld * m;
-    int32_t* d_reps = nullptr;
-    auto factor = [&](std::vector<int32_t>& piv) -> int {
-      if (!alloc(&V->lu, ts * nc * V->lstride) || !alloc((void**)&V->rdiag, sizeof(double) * nc * m) ||
-          !alloc((void**)&d_reps, sizeof(int32_t) * nc * (1 + m)))
+    const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
+    // Factors of the classes, and beside them the comparison of the patches with
+    // their firsts; hashes that agreed by chance make one more turn.
+    auto factor = [&]() -> int {
+      const int64_t nc = V->nclasses = (int64_t)reps.size();
+      const size_t lub = ts * nc * V->lstride;
+      if (V->lu) (void)hipFree(V->lu);
+      V->lu = nullptr;
+      if (hipMalloc(&V->lu, lub + sizeof(double) * nc * m) != hipSuccess)
         return fail(GH_ENOMEM, "gh_vanka_create: allocation failed");
-      int32_t* d_piv = d_reps + nc;
-      GH_HIP(hipMemcpyAsync(d_reps, reps.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice,
+      V->rdiag = (double*)((char*)V->lu + lub);
+      int32_t *d_piv = (int32_t*)V->xp, *d_first = d_piv + nc * m, *d_differs = d_first + np;
+      std::vector<int32_t> up(cls);
+      up.insert(up.end(), reps.begin(), reps.end());
+      GH_HIP(hipMemcpyAsync(V->cls, up.data(), sizeof(int32_t) * up.size(), hipMemcpyHostToDevice,
                             ctx->stream));
-      GH_HIP(hipMemcpyAsync(V->cls, cls.data(), sizeof(int32_t) * npatches, hipMemcpyHostToDevice,
-                            ctx->stream));
-      GH_HIP(hipMemsetAsync(V->lu, 0, ts * nc * V->lstride, ctx->stream));
-      const size_t lds = sizeof(int32_t) * (size_t)psize * psize;
       GH_HIP(hipFuncSetAttribute((const void*)k_vanka_factor,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
       hipLaunchKernelGGL(k_vanka_factor, dim3((unsigned)nc), dim3(kFactorThreads), lds, ctx->stream,
@@ -1012,20 +1016,35 @@ int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, cons
         hipLaunchKernelGGL(k_vanka_rdiag<float>, gr, dim3(kBlock), 0, ctx->stream, nc, m,
                            V->ld, (const float*)V->lu, V->rdiag);
       GH_HIP(hipGetLastError());
-      piv.resize((size_t)nc * m);
+      const bool compare = nc < np;
+      if (compare) {
+        GH_HIP(hipMemcpyAsync(d_first, first.data(), sizeof(int32_t) * np, hipMemcpyHostToDevice,
+                              ctx->stream));
+        GH_HIP(hipFuncSetAttribute((const void*)k_vanka_same,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * lds)));
+        hipLaunchKernelGGL(k_vanka_same, dim3((unsigned)np), dim3(kHashThreads), 2 * lds, ctx->stream,
+                           psize, B, V->nodes, A->rowptr, A->col, (const double*)A->val, d_first,
+                           d_differs);
+        GH_HIP(hipGetLastError());
+      }
+      piv.resize((size_t)nc * m + (compare ? 2 * np : 0));
       GH_HIP(hipMemcpyAsync(piv.data(), d_piv, sizeof(int32_t) * piv.size(), hipMemcpyDeviceToHost,
                             ctx->stream));
       GH_HIP(hipStreamSynchronize(ctx->stream));
       return GH_OK;
     };
-    std::vector<int32_t> piv;
-    const int frc = factor(piv);
-    if (d_reps) (void)hipFree(d_reps);
-    if (frc) return bail(frc);
+    for (;;) {
+      patch_classes(first, differs, cls, reps);
+      if (int rc = factor()) return bail(rc);
+      const int64_t nc = V->nclasses;
+      if (nc == np || std::equal(differs.begin(), differs.end(), piv.begin() + nc * m + np)) break;
+      differs.assign(piv.begin() + nc * m + np, piv.end());
+    }
+    const int64_t nc = V->nclasses;
     // Compose the recorded row exchanges (applied in order k = 0..m-1) into
     // one gather: row i of P h is local entry src[i], i.e. the global entry
     // node(src[i] / B) * B + src[i] % B.  The solve then needs no exchanges.
-    std::vector<int32_t> src((size_t)nc * m), gidx((size_t)npatches * m);
+    std::vector<int32_t> src((size_t)nc * m), lists((size_t)np * m), plist, groups;
     for (int64_t c = 0; c < nc; ++c) {
       const int32_t* pv = piv.data() + c * m;
       int32_t* sc = src.data() + c * m;
@@ -1035,16 +1054,18 @@ int vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize, cons
         std::swap(sc[k], sc[pv[k]]);
       }
     }
-    parallel_for(npatches, 2048, [&](int64_t a, int64_t b) {
+    parallel_for(np, 2048, [&](int64_t a, int64_t b) {
       for (int64_t p = a; p < b; ++p) {
         const int32_t* sc = src.data() + (int64_t)cls[p] * m;
         for (int i = 0; i < m; ++i)
-          gidx[p * m + i] = (int32_t)((int64_t)nodes[p * psize + sc[i] / B] * B + sc[i] % B);
+          lists[p * m + i] = (int32_t)((int64_t)nodes[p * psize + sc[i] / B] * B + sc[i] % B);
       }
     });
-    if (hipMemcpy(V->piv, gidx.data(), sizeof(int32_t) * gidx.size(), hipMemcpyHostToDevice) != hipSuccess)
+    vanka_groups(ctx, V, cls, plist, groups);
+    lists.insert(lists.end(), plist.begin(), plist.end());
+    lists.insert(lists.end(), groups.begin(), groups.end());
+    if (hipMemcpy(V->piv, lists.data(), sizeof(int32_t) * lists.size(), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(GH_EHIP, "gh_vanka_create: gather upload failed"));
-    if (int rc = vanka_groups(ctx, V, cls)) return bail(rc);
   }
   *out = V;
   return GH_OK;
@@ -1064,8 +1085,7 @@ int gh_vanka_create(gh_ctx* ctx, const gh_csr* A, int64_t npatches, int psize,
 int gh_vanka_destroy(gh_vanka* V) {
   if (!V) return GH_OK;
   if (V->ctx && V->ctx->stream) (void)hipStreamSynchronize(V->ctx->stream);
-  for (void* p : {(void*)V->nodes, (void*)V->cls, V->lu, (void*)V->rdiag, (void*)V->piv,
-                  (void*)V->nptr, (void*)V->nent, V->xp, (void*)V->groups, (void*)V->plist})
+  for (void* p : {(void*)V->ints, V->lu, V->xp})
     if (p) (void)hipFree(p);
   gh_ctx* ctx = V->ctx;
   delete V;
