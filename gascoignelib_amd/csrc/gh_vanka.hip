@@ -839,11 +839,13 @@ void patch_classes(const std::vector<int32_t>& first, const std::vector<int32_t>
 }
 
 // Whether the grouped solve runs, and its groups: chunks of a class's patches, as
-// many per workgroup as make the solve shortest.  A workgroup stages its factors
-// (taken as long as one pass) and then solves 32 patches per pass; workgroups
-// beyond those the chip holds at once wait for a place.  (32768 patches of 108
-// unknowns in 27 classes, FP64, one workgroup per CU: 128 patches each would be 270
-// workgroups and a second round for the last 14.)
+// many per workgroup as make the solve shortest.  A CU works off its share of the
+// workgroups, `fit` at a time; they take their patches' LDS reads and issue one
+// after the other, with the staging on top, but not less than the chain of 2 m
+// steps, which is as long as the work of 24 patches at m = 108 and of more where a
+// patch is smaller.  108 unknowns, FP64 (FP32), copy and averaging included: 32768
+// patches in 68 classes, 72 to a workgroup 124 us (75), 128 187 (109), 32 147 (74),
+// 8 292 (103); 4096 patches, 20 to a workgroup 36 (26), 8 61 (28), 64 55 (39).
 //
 // Against the streamed solve the groups must hold enough patches for the factors
 // staged: with one patch each they are slower for any number of patches (108
@@ -866,21 +868,27 @@ void vanka_groups(gh_ctx* ctx, gh_vanka* V, const std::vector<int32_t>& cls,
   std::vector<int64_t> start(nc + 1, 0);
   for (int64_t p = 0; p < np; ++p) start[cls[p] + 1]++;
   const int64_t most = *std::max_element(start.begin(), start.end());
-  constexpr int64_t kPass = kGroupThreads / 16;  // patches per pass
-  const int64_t least = V->m > 64 ? 3 : 2;       // patches per group
-  int64_t chunk = 0, ng = 0, best = 0;
-  for (int64_t c = 4;; c += c < kPass ? 4 : kPass) {  // a wavefront takes 4 patches
+  const int64_t least = V->m > 64 ? 3 : 2;  // patches per group
+  const int64_t cu = ctx->num_cu;
+  const double stage = 8.0, chain = 24.0 * 108.0 / V->m;  // in patches
+  auto time = [&](int64_t groups, int64_t c) {  // of the CU that has the most groups
+    const int64_t share = (groups + cu - 1) / cu, full = share / fit, rest = share % fit;
+    return (double)full * std::max(chain, (double)(fit * c) + stage) +
+           (rest ? std::max(chain, (double)(rest * c) + stage) : 0.0);
+  };
+  int64_t chunk = 0, ng = 0;
+  double best = 0.0;
+  for (int64_t c = 4;; c += 4) {  // a wavefront takes 4 patches
     int64_t g = 0;
     for (int64_t k = 1; k <= nc; ++k) g += (start[k] + c - 1) / c;
-    const int64_t cost = ((g + at_once - 1) / at_once) * (1 + (c + kPass - 1) / kPass);
+    const double cost = time(g, c);
     if (chunk == 0 || cost < best || (cost == best && np < least * ng)) {
       chunk = c;
       ng = g;
       best = cost;
     }
-    // no larger chunk is shorter: one group per class is the least there can be
-    const int64_t rounds = (nc + at_once - 1) / at_once;
-    if (c >= most || (g <= at_once && np >= least * g) || rounds * (2 + c / kPass) > best) break;
+    // one group per class is the least there can be
+    if (c >= most || time(nc, c) > best) break;
   }
   if (np < least * ng || (ng > at_once && np * fit < (least + 2) * ng)) return;
   for (int64_t c = 0; c < nc; ++c) start[c + 1] += start[c];
