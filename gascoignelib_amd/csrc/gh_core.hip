@@ -862,6 +862,16 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
     GH_HIP(hipStreamSynchronize(ctx->stream));
     return GH_OK;
   }
+  {
+    std::vector<uint8_t> down(ns, 0);
+    parallel_for(ns, 512, [&](int64_t s0, int64_t s1) {
+      for (int64_t s = s0; s < s1; ++s)
+        for (int64_t i = s * kSlice; i < std::min<int64_t>(n, (s + 1) * kSlice) && !down[s]; ++i)
+          for (int64_t q = rowptr[i] + 1; q < rowptr[i + 1] && !down[s]; ++q)
+            down[s] = col[q] < col[q - 1];
+    });
+    S->ascending = std::find(down.begin(), down.end(), 1) == down.end();
+  }
   // Relative column patterns (col - row over a row's kept entries, in order)
   // that at least kMinPatternRows rows share.  A slice whose rows all follow
   // table patterns stores no columns: rlen holds the pattern ids.

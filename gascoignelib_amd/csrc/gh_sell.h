@@ -681,13 +681,18 @@ __global__ __launch_bounds__(kSlice * K) void k_sell_fold(
 //    then wait for nothing: rows of 27 and 96, 120 K rows 14.3 / 17.3 / 23.0 against
 //    19.2 / 17.6 / 23.0 with columns in memory.  Where they hold most of the entries,
 //    the fold is for few slices only.
+//  * Ascending columns gather from fewer lines than a caller's order, and enough
+//    slices hide what is left: Q2 with hanging nodes, 352 K rows 86 / 56 against
+//    109 / 61 in the caller's order, but 1.96 M rows (30.7 K slices) 303 / 331
+//    against 400 / 360, and A z with an FP32 z 294 / 349.
 constexpr int kFoldRow = 32, kFoldLong = 64;
-constexpr int64_t kFoldSlices4 = 512;
+constexpr int64_t kFoldSlices4 = 512, kFoldSlicesAscending = 16384;
 inline int sell_fold_waves(const Sell& S) {
   if (S.maxlen <= kFoldRow) return 0;
   if (S.nslices <= 5 * (int64_t)S.maxlen) return 8;
   if (2 * S.single > S.slots) return 0;
   if (S.nslices <= kFoldSlices4) return 4;
+  if (S.ascending && S.nslices > kFoldSlicesAscending) return 0;
   return S.maxlen > kFoldLong && 2 * S.nslices * S.maxlen * kSlice >= 3 * S.slots ? 4 : 0;
 }
 

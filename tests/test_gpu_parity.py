@@ -697,14 +697,16 @@ def mixed_rows(n, L, share, short, columns, seed):
 
 # few slices (5 per entry of the longest row) take 8 wavefronts, up to 512 take 4;
 # more only where rows of more than 64 entries are 1.5 times the mean and most
-# entries lie outside single-pattern slices
+# entries lie outside single-pattern slices, up to 16384 if the columns ascend (as
+# in every matrix from the caller)
 @pytest.mark.parametrize("n,L,share,short,columns,waves", [
     (640, 32, 1.0, 32, "random", 8), (640, 31, 1.0, 31, "random", 1),
     (5000, 40, 1.0, 40, "band", 8), (10000, 33, 0.5, 9, "random", 8),
     (12000, 36, 0.1, 27, "random", 4), (12000, 36, 1.0, 36, "band", 1),
     (32768, 60, 0.5, 27, "random", 4), (32769, 60, 0.5, 27, "random", 1),
     (50000, 51, 0.05, 18, "random", 1), (50000, 100, 0.25, 9, "random", 4),
-    (50000, 100, 0.25, 9, "band", 1), (50000, 100, 1.0, 100, "random", 1)])
+    (50000, 100, 0.25, 9, "band", 1), (50000, 100, 1.0, 100, "random", 1),
+    (1048576, 66, 0.05, 2, "random", 4), (1048577, 66, 0.05, 2, "random", 1)])
 def test_fp64_sweep_forms(ctx, n, L, share, short, columns, waves):
     """each matrix takes the form of the FP64 sweep that is faster for it, and
     every form keeps the oracle's bits"""
