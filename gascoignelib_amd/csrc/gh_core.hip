@@ -862,7 +862,8 @@ static int sell_build_impl(gh_ctx* ctx, int64_t n, const int32_t* rowptr, const 
     GH_HIP(hipStreamSynchronize(ctx->stream));
     return GH_OK;
   }
-  {
+  S->ascending = false;
+  if (S->maxlen > kFoldRow) {  // (looked at by sell_fold_waves only)
     std::vector<uint8_t> down(ns, 0);
     parallel_for(ns, 512, [&](int64_t s0, int64_t s1) {
       for (int64_t s = s0; s < s1; ++s)

@@ -156,7 +156,7 @@ struct Sell {
   int64_t stored = 0;     // entries kept (valued operators drop exact zeros)
   int64_t narrow = 0;     // slices with 16-bit column offsets
   int maxlen = 0;         // longest row (entries kept)
-  bool ascending = false;  // every row's columns ascend (valued operators)
+  bool ascending = false;  // every row's columns ascend (valued operators with rows > 32)
   uint32_t* sptr = nullptr;  // nslices+1 slot offsets
   uint16_t* rlen = nullptr;  // entries per row
   // valued operators, per slice one of three column encodings:
