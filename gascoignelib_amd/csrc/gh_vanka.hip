@@ -625,9 +625,10 @@ __host__ __device__ constexpr int group_entries(int mb) { return 256 * mb * mb; 
 // broadcast to the 16 lanes by one DPP move per half.  A wavefront thus solves 4
 // patches at a time with the LDS reads shared between them; every entry sees the
 // operations of k_vanka_solve in the same order.  Bound by the chain of 2 m
-// dependent steps, not by memory: 108 unknowns, 4096 patches in 68 classes, 20.6
-// us in FP32 and 37.8 in FP64 (k_vanka_solve: 56 and 107), 512 patches 13.3 and
-// 17.2 (36 and 40).
+// dependent steps while a CU has few patches, then by their LDS reads and issue,
+// not by memory: 108 unknowns, 68 classes, 512 patches 13.9 us in FP32 and 17.4 in
+// FP64 (one wavefront and one set of factors per patch 36 and 40), 4096 18.6 and
+// 26.6 (56 and 107), 32768 60 and 105.
 constexpr int kGroupThreads = 512;
 template <typename T, int MB>
 __global__ __launch_bounds__(kGroupThreads) void k_vanka_group(int m, int64_t lstride,
